@@ -14,17 +14,27 @@
 // column pair with everything but padding, padding pairs only with itself, and the size
 // vectors gain (valid_text, text - valid_text).
 //
-// Layout: a workgroup of kSelWaves waves owns kSelWaves query rows of one batch entry and
-// streams the key centroids through LDS in blocks of 64 rows (row stride dims+1 floats, so
-// lane j reading row j is bank-conflict free), with up to four blocks in flight in registers
-// (at 480p 10% faster than one); lane j of a wave scores key j of the block.
-// Each wave then holds its row's ck keys in registers, KPL = ck_pow2/64 per lane, and sorts
-// them with a register bitonic network (cross-lane stages by xor shuffles).
+// Layout: a workgroup of kSelWaves waves owns kSelWaves query rows of one batch entry.
+// Scores: the key centroids stream through LDS in chunks of (up to 512 keys) x (C channels), so a
+// key value is read from LDS once per workgroup row group instead of once per row: a wave holds two
+// keys per lane and up to four query rows (8 independent fma chains). The finished dots go through
+// LDS to the row layout: wave = row, lane l holds keys l, l + 64, ...
 //
 // The kept set is a prefix of the sorted order: with probabilities descending and the
 // running sum nondecreasing, cum_{k+1} - prob_{k+1} >= cum_k - prob_k exactly, so the
-// rounded `before` values are nondecreasing too. The sequential double walk therefore
-// stops at the first entry past the minimum whose `before` reaches p.
+// rounded `before` values are nondecreasing too. So the row is not sorted: a binary search over
+// the probability bits finds the value v at which the prefix ends (every lane holds its keys, a
+// step is a count by ballots and one wave sum), and the decision at the boundary is then made on
+// the reference's own quantities. The cumulative sum enters only as fl32(cum): with D the double
+// sum (in any order) of the prefix, |D - cum| < kCumEps, so when D - kCumEps and D + kCumEps
+// decide alike, the sequential sum decides so too. Checked are the last entry above v (must be
+// kept), every entry equal to v (in index order) and, when all of those are kept, the first
+// entry below (must not be). A boundary the float sums of the search placed one value off is moved;
+// a decision that stays open, or a row with non-finite mass, takes the sequential walk itself.
+// Bound by latency: a few dependent phases of one to two workgroups per CU. Launch times (work-list
+// form, 128 channels; before: one wave per row reading every key row from LDS for itself, a sort of
+// 64-bit keys, the sequential walk, 196 VGPRs and so one workgroup per CU): 24 heads x 64 rows x
+// 256 keys 27 us (37 before), 100 x 500 43 us (102), 128 x 512 52 us (113), 256 x 1024 147 us (366).
 #include "common.hpp"
 #include "work.hpp"
 
@@ -38,15 +48,24 @@ constexpr int kSelWaves = 8;
 constexpr int kSelThreads = kSelWaves * kWave;
 constexpr int kSelBlock = 64;
 constexpr int kSelMaxDims = 256;
-// Staged floats per thread and key block: kWide (dims up to kSelMaxDims) or not (up to 128).
-template <bool kWide> constexpr int sel_loads() { return kSelBlock * (kWide ? kSelMaxDims : 128) / kSelThreads; }
-// Key blocks in flight: 64 staged floats per thread (32 when each lane also holds 16 or more
-// keys, whose registers the row needs), at most the blocks there are.
-template <int KPL, bool kWide> constexpr int sel_depth() {
-    const int d = (KPL >= 16 ? 32 : 64) / sel_loads<kWide>();
-    return d < 1 ? 1 : (d > KPL ? KPL : d);
-}
-constexpr int kSelBatch = 32;
+constexpr int kSelStage = 16;  // staged floats per thread and chunk
+
+// Shapes of the score phase for KPL keys per lane of a row.
+template <int KPL> struct SelTiles {
+    static constexpr int kBlocks = KPL < 8 ? KPL : 8;              // 64-key blocks per pass
+    static constexpr int kPasses = KPL / kBlocks;
+    static constexpr int kKeys = kSelBlock * kBlocks;              // keys per pass
+    static constexpr int kChan = kSelStage * kSelThreads / kKeys;  // channels per chunk
+    static constexpr int kStride = kChan + 1;                      // LDS row (odd: lanes on distinct banks)
+    static constexpr int KW = KPL < 2 ? 1 : 2;                     // keys per lane of the score phase
+    static constexpr int kGroups = kBlocks / KW;                   // key groups, one wave each per row set
+    static constexpr int kRows = kGroups;                          // query rows per wave
+    static constexpr size_t kLdsFloats = static_cast<size_t>(kKeys) * kStride + static_cast<size_t>(kSelWaves) * kKeys;
+};
+
+// Bound of |double sum of at most 2048 probabilities in any order - the sequential one| (each at
+// most 2048 * 2^-53 of a sum near 1).
+constexpr double kCumEps = 9.094947017729282e-13;  // 2^-40
 
 __device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int mask) {
     const int lo = __shfl_xor(static_cast<int>(static_cast<uint32_t>(v)), mask, kWave);
@@ -58,6 +77,224 @@ __device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int mask) {
 __device__ __forceinline__ float key_prob(uint32_t high) {
     const uint32_t ord = ~high;
     return __uint_as_float((ord & 0x80000000u) ? (ord & 0x7fffffffu) : ~ord);
+}
+
+// Lane exchange inside a 16-lane row. The four levels pair each lane with a lane of the other half
+// of its group of 2, 4, 8 and 16; every lane of a half holds the half's result, so a reduction by
+// these levels equals the xor-shuffle tree.
+template <int kLevel> __device__ __forceinline__ int row_pair(int v) {
+    constexpr int kCtrl = kLevel == 0 ? 0xb1 : kLevel == 1 ? 0x4e : kLevel == 2 ? 0x141 : 0x140;
+    return __builtin_amdgcn_update_dpp(v, v, kCtrl, 0xf, 0xf, false);
+}
+
+template <typename Op> __device__ __forceinline__ float wave_reduce_f32(float v, Op op) {
+    auto pair = [](int x) { return __int_as_float(x); };
+    v = op(v, pair(row_pair<0>(__float_as_int(v))));
+    v = op(v, pair(row_pair<1>(__float_as_int(v))));
+    v = op(v, pair(row_pair<2>(__float_as_int(v))));
+    v = op(v, pair(row_pair<3>(__float_as_int(v))));
+    v = op(v, __shfl_xor(v, 16, kWave));
+    return op(v, __shfl_xor(v, 32, kWave));
+}
+
+// The same for values whose order of combination does not matter (all lanes of a row hold the row's
+// result after the four levels; the rows are then read as scalars).
+template <typename Op> __device__ __forceinline__ int wave_reduce_i32(int v, Op op) {
+    v = op(v, row_pair<0>(v));
+    v = op(v, row_pair<1>(v));
+    v = op(v, row_pair<2>(v));
+    v = op(v, row_pair<3>(v));
+    const int a = op(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16));
+    return op(a, op(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+}
+
+__device__ __forceinline__ float lane_f32(float v, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+
+__device__ __forceinline__ float wave_sum_any(float v) {
+    v += __int_as_float(row_pair<0>(__float_as_int(v)));
+    v += __int_as_float(row_pair<1>(__float_as_int(v)));
+    v += __int_as_float(row_pair<2>(__float_as_int(v)));
+    v += __int_as_float(row_pair<3>(__float_as_int(v)));
+    return (lane_f32(v, 0) + lane_f32(v, 16)) + (lane_f32(v, 32) + lane_f32(v, 48));
+}
+
+__device__ __forceinline__ double wave_sum_f64(double v) {
+#pragma unroll
+    for (int m = 1; m < kWave; m <<= 1) v += __longlong_as_double(shfl_xor_u64(__double_as_longlong(v), m));
+    return v;
+}
+
+// Whether entry k of the descending order (probability prob, cumulative sum cum up to and with it)
+// is kept: 1 or 0, or -1 when the two ends of the cumulative sum's error band decide differently.
+__device__ __forceinline__ int keep_decision(int k, int floor_keep, double cum, float prob, float p) {
+    if (k < floor_keep) return 1;
+    const bool lo = static_cast<float>(cum - kCumEps) - prob < p;
+    const bool hi = static_cast<float>(cum + kCumEps) - prob < p;
+    return lo == hi ? (lo ? 1 : 0) : -1;
+}
+
+// The kept prefix of one row by the sequential definition: entries in descending order (ties by
+// index) until one past the minimum fails. Slot e of lane l is key 64 e + l; bit e of the result: slot
+// e kept. Taken by rows with non-finite mass and by decisions the search leaves open.
+template <int KPL>
+__device__ __forceinline__ uint32_t keep_sequential(const float (&prob)[KPL], int ck, int floor_keep, float p) {
+    const int lane = lane_id();
+    uint32_t keep = 0;
+    uint64_t last = 0;
+    double run = 0.0;
+    for (int k = 0; k < ck; ++k) {
+        // Smallest sort key (~orderable(prob), index) past the last one.
+        uint64_t best = ~0ull;
+#pragma unroll
+        for (int e = 0; e < KPL; ++e) {
+            const int j = e * kSelBlock + lane;
+            const uint64_t key = (static_cast<uint64_t>(~orderable(prob[e])) << 32) | static_cast<uint32_t>(j);
+            if (j < ck && (k == 0 || key > last) && key < best) best = key;
+        }
+#pragma unroll
+        for (int m = 1; m < kWave; m <<= 1) {
+            const uint64_t other = shfl_xor_u64(best, m);
+            best = other < best ? other : best;
+        }
+        const float pr = key_prob(static_cast<uint32_t>(best >> 32));
+        run += static_cast<double>(pr);
+        if (k >= floor_keep && !(static_cast<float>(run) - pr < p)) break;
+        last = best;
+        const int j = static_cast<int>(best & 0xffffffffu);
+        if (lane == j % kSelBlock) keep |= 1u << (j / kSelBlock);
+    }
+    return keep;
+}
+
+// The same by search (see the head of the file); bit e of the result: slot e kept. False when a
+// decision at the boundary stays open.
+template <int KPL>
+__device__ __forceinline__ bool keep_search(const float (&prob)[KPL], int ck, int floor_keep, float p, uint32_t& result) {
+    const int lane = lane_id();
+    int u[KPL];  // probability bits, ordered as integers; below 0 for an absent key (probability -1)
+#pragma unroll
+    for (int e = 0; e < KPL; ++e) u[e] = __float_as_int(prob[e]);
+    // Entries with bits above v: their count and mass.
+    auto above = [&](int v, int& n, float& mass) __attribute__((always_inline)) {
+        float part = 0.0f;
+        n = 0;
+#pragma unroll
+        for (int e = 0; e < KPL; ++e) {
+            const bool g = u[e] > v;
+            n += __popcll(__ballot(g));
+            part += g ? prob[e] : 0.0f;
+        }
+        mass = wave_sum_any(part);
+    };
+    auto imax = [](int a, int b) { return max(a, b); };
+    auto imin = [](int a, int b) { return min(a, b); };
+    // The entry after those above v is kept when it is within the minimum or their mass is below p;
+    // v: the smallest bits for which that holds (lo: a value it does not hold for).
+    int v = u[0];
+#pragma unroll
+    for (int e = 1; e < KPL; ++e) v = max(v, u[e]);
+    v = wave_reduce_i32(v, imax);
+    int lo = -1, n_lo = ck, n_hi = 0;
+    {
+        int n;
+        float mass;
+        above(lo, n, mass);
+        if (mass < p) v = lo;  // (all ck entries are past the minimum)
+    }
+    while (v - lo > 1) {
+        const int mid = lo + ((v - lo) >> 1);
+        int n;
+        float mass;
+        above(mid, n, mass);
+        if (n < floor_keep || mass < p) {
+            v = mid;
+            n_hi = n;
+        } else {
+            lo = mid;
+            n_lo = n;
+        }
+        if (n_lo - n_hi == 1) {  // one entry in (lo, v]: the value sought is its own
+            int best = -1;
+#pragma unroll
+            for (int e = 0; e < KPL; ++e) best = u[e] <= v ? max(best, u[e]) : best;
+            v = wave_reduce_i32(best, imax);
+            break;
+        }
+    }
+    for (int moves = 0; moves < 4; ++moves) {
+        double part = 0.0;
+        int n = 0, least = 0x7fffffff, below = -1;
+        uint32_t keep = 0;
+#pragma unroll
+        for (int e = 0; e < KPL; ++e) {
+            const bool g = u[e] > v;
+            n += __popcll(__ballot(g));
+            part += g ? static_cast<double>(prob[e]) : 0.0;
+            least = g ? min(least, u[e]) : least;
+            below = u[e] < v ? max(below, u[e]) : below;
+            keep |= g ? 1u << e : 0u;
+        }
+        const double cum = wave_sum_f64(part);
+        least = wave_reduce_i32(least, imin);
+        below = wave_reduce_i32(below, imax);
+        if (n > 0) {
+            const int d = keep_decision(n - 1, floor_keep, cum, __int_as_float(least), p);
+            if (d < 0) return false;
+            if (d == 0) {
+                v = least;
+                continue;
+            }
+        }
+        // Entries equal to v, in index order.
+        const float value = __int_as_float(max(v, 0));
+        int ties = 0;
+        bool open = false, failed = false;
+#pragma unroll
+        for (int e = 0; e < KPL; ++e) {
+            const bool q = u[e] == v && v >= 0;
+            const uint64_t m = __ballot(q);
+            if (m == 0) continue;
+            const int rank = ties + static_cast<int>(__builtin_amdgcn_mbcnt_hi(
+                                        static_cast<uint32_t>(m >> 32),
+                                        __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0)));
+            const int d = keep_decision(n + rank, floor_keep,
+                                        cum + static_cast<double>(rank + 1) * static_cast<double>(value), value, p);
+            open = open || (q && d < 0);
+            failed = failed || (q && d == 0);
+            keep |= q && d > 0 ? 1u << e : 0u;
+            ties += __popcll(m);
+        }
+        if (__any(open)) return false;
+        if (!__any(failed) && below >= 0) {
+            const float next = __int_as_float(below);
+            const int d = keep_decision(
+                n + ties, floor_keep,
+                cum + static_cast<double>(ties) * static_cast<double>(value) + static_cast<double>(next), next, p);
+            if (d < 0) return false;
+            if (d > 0) {
+                v = below;
+                continue;
+            }
+        }
+        result = keep;
+        return true;
+    }
+    return false;
+}
+
+template <int KPL>
+__device__ __forceinline__ uint32_t keep_prefix(const float (&prob)[KPL], int ck, int floor_keep, float p, bool finite) {
+    const int lane = lane_id();
+    uint32_t keep = 0;
+#pragma unroll
+    for (int e = 0; e < KPL; ++e)
+        if (e * kSelBlock + lane < ck) keep |= 1u << e;
+    if (p >= 1.0f || ck <= floor_keep) return keep;
+    if (!finite || !keep_search<KPL>(prob, ck, floor_keep, p, keep))
+        keep = keep_sequential<KPL>(prob, ck, floor_keep, p);
+    return keep;
 }
 
 // Kept-segment list of one map row, written by one wavefront: lane l takes clusters l,
@@ -83,7 +320,7 @@ __device__ int write_segments(int2* __restrict__ srow, const int (&kcnt)[KPL], i
         const int incl = wave_incl_scan(size);
         const int a = min(sk, pre + incl - size), e = min(sk, pre + incl);
         const bool has_rows = e > a;
-        const bool on = has_rows && kept(j);
+        const bool on = has_rows && kept(j, ch);
         const uint64_t with_rows = __ballot(has_rows), on_mask = __ballot(on);
         const uint64_t lower = with_rows & below;
         const bool prev = lower ? ((on_mask >> (63 - __builtin_clzll(lower))) & 1ull) != 0 : prev_on;
@@ -94,8 +331,8 @@ __device__ int write_segments(int2* __restrict__ srow, const int (&kcnt)[KPL], i
         const int off = run + oincl - orows;  // stream offset of cluster j
         if (start) srow[1 + nseg + __popcll(starts & below)] = int2{a - off, off};
         nseg += __popcll(starts);
-        run += __shfl(oincl, kWave - 1, kWave);
-        pre += __shfl(incl, kWave - 1, kWave);
+        run += __builtin_amdgcn_readlane(oincl, kWave - 1);
+        pre += __builtin_amdgcn_readlane(incl, kWave - 1);
         if (with_rows) prev_on = ((on_mask >> (63 - __builtin_clzll(with_rows))) & 1ull) != 0;
     }
     if (lane == 0) {
@@ -108,14 +345,16 @@ __device__ int write_segments(int2* __restrict__ srow, const int (&kcnt)[KPL], i
 // kWork: besides (or instead of) the map, write every map row's kept-segment list and stream
 // length into `work`; the last workgroup of each batch entry to finish (arrival counter) then
 // orders that entry's attention items.
-template <int KPL, bool kWork, bool kWide>
-__global__ __launch_bounds__(kSelWaves * kWave) void select_kernel(
+template <int KPL, bool kWork>
+__global__ __launch_bounds__(kSelThreads, KPL > 16 ? 2 : 4) void select_kernel(
     const float* __restrict__ qc, const float* __restrict__ kc, const int32_t* __restrict__ qn,
     const int32_t* __restrict__ kn, int bh, int cq, int ck, int dims, float scale, float p, int minimum, int extend,
     int valid_text, int text, uint8_t* __restrict__ map, int32_t* __restrict__ ext_q, int32_t* __restrict__ ext_k,
     int32_t* __restrict__ kept_keys, int sq, int sk, SelWork work) {
     extern __shared__ __align__(16) unsigned char smem[];
-    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    using T = SelTiles<KPL>;
+    const int lane = threadIdx.x % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int groups = static_cast<int>(ceil_div(cq, kSelWaves));
     const int b = blockIdx.x / groups;
     const int c0 = (blockIdx.x % groups) * kSelWaves;
@@ -123,11 +362,10 @@ __global__ __launch_bounds__(kSelWaves * kWave) void select_kernel(
     const bool active = c < cq;
     const int ce = extend ? ck + 2 : ck;
     const int re = extend ? cq + 2 : cq;
-    const int kstride = dims + 1;
-    const int qstride = (dims + 3) & ~3;                    // keeps float4 reads of a row aligned
-    float* qrows = reinterpret_cast<float*>(smem);          // [kSelWaves][qstride]
-    float* kblk = qrows + kSelWaves * qstride;               // [kSelBlock][dims + 1]
-    uint8_t* flags = reinterpret_cast<uint8_t*>(kblk + kSelBlock * kstride) + static_cast<size_t>(wave) * ck;
+    const int qstride = (dims + 3) & ~3;             // keeps float4 reads of a row aligned
+    float* qrows = reinterpret_cast<float*>(smem);   // [kSelWaves][qstride]
+    float* kblk = qrows + kSelWaves * qstride;        // [kKeys][kStride] one chunk of the keys
+    float* dots = kblk + T::kKeys * T::kStride;       // [kSelWaves][kKeys] a pass's scores, by row
 
     // Text partition rows and extended sizes (once per batch entry).
     if (extend && c0 == 0 && wave == 0) {
@@ -166,204 +404,150 @@ __global__ __launch_bounds__(kSelWaves * kWave) void select_kernel(
         qrows[(t / dims) * qstride + t % dims] = r < cq ? qc[(static_cast<int64_t>(b) * cq + r) * dims + t % dims] : 0.0f;
     }
     const int32_t* kcount = kn + static_cast<int64_t>(b) * ck;
-    const float* q = qrows + wave * qstride;
 
-    // Key blocks are fetched into registers kDepth blocks ahead (all loads of a block in flight
-    // at once) and stored to LDS rows of stride dims+1. Thread t handles elements t, t + 512, ...
-    // of the block; (row, col) of element t advance incrementally.
-    constexpr int kLoads = sel_loads<kWide>();
-    constexpr int kDepth = sel_depth<KPL, kWide>();
-    float staged[kDepth][kLoads];
-    const int row_step = kSelThreads / dims, col_step = kSelThreads % dims;
-    const int row0 = threadIdx.x / dims, col0 = threadIdx.x % dims;
-    auto fetch = [&](float (&dst)[kLoads], int base) {
-        const int n = min(kSelBlock, ck - base) * dims;
-        const float* src = kc + (static_cast<int64_t>(b) * ck + base) * dims;
+    // A chunk goes through registers: kSelStage floats per thread, all loads in flight (clamped, so
+    // unconditional), requested while the chunk before is used.
+    float staged[kSelStage];
+    const int chunks = static_cast<int>(ceil_div(dims, T::kChan));
+    const char* keys_bytes = reinterpret_cast<const char*>(kc + static_cast<int64_t>(b) * ck * dims);
+    const int srow = threadIdx.x / T::kChan, scol = threadIdx.x % T::kChan;
+    constexpr int kRowStep = kSelThreads / T::kChan;
+    auto fetch = [&](int pass, int chunk) {
+        const int col = min(chunk * T::kChan + scol, dims - 1);
 #pragma unroll
-        for (int v = 0; v < kLoads; ++v) {
-            const int t = v * kSelThreads + static_cast<int>(threadIdx.x);
-            dst[v] = src[min(t, n - 1)];  // unconditional (clamped): all loads in flight
+        for (int i = 0; i < kSelStage; ++i) {
+            const int row = min(pass * T::kKeys + srow + i * kRowStep, ck - 1);
+            // 32-bit byte offsets from the uniform base: ck <= 2048 rows of at most 256 channels.
+            staged[i] = *reinterpret_cast<const float*>(keys_bytes + static_cast<uint32_t>(row * dims + col) * 4u);
         }
     };
-    auto store = [&](const float (&src)[kLoads], int base) {
-        const int n = min(kSelBlock, ck - base) * dims;
-        int row = row0, col = col0;
+    // Score phase: this wave's key group and first query row.
+    const int kg = wave % T::kGroups, r0 = (wave / T::kGroups) * T::kRows;
+    int kcnt[KPL];      // counts of keys 64 e + lane (0 past ck)
+    float prob[KPL];    // dot products, then logits, masses and probabilities
+    fetch(0, 0);
 #pragma unroll
-        for (int v = 0; v < kLoads; ++v) {
-            if (v * kSelThreads + static_cast<int>(threadIdx.x) < n) kblk[row * kstride + col] = src[v];
-            row += row_step;
-            col += col_step;
-            if (col >= dims) {
-                col -= dims;
-                ++row;
-            }
-        }
-    };
-
-    // Logits of key j = 64 e + lane in register slot e. The slots first hold log(count_j)
-    // (-inf for an empty or absent key), read before any key block is prefetched.
-    float logit[KPL];
-    int kcnt[KPL];  // the counts again, for the segment lists
+    for (int pass = 0; pass < T::kPasses; ++pass) {
+        if (pass > 0 && pass * T::kKeys >= ck) break;
+        float acc[T::kRows][T::KW];
 #pragma unroll
-    for (int e = 0; e < KPL; ++e) {
-        const int j = e * kSelBlock + lane;
-        const int wl = kcount[min(j, ck - 1)];
-        const int w = j < ck ? wl : 0;
-        kcnt[e] = max(0, w);
-        logit[e] = w > 0 ? logf(static_cast<float>(w)) : -INFINITY;
-    }
+        for (int r = 0; r < T::kRows; ++r)
 #pragma unroll
-    for (int e = 0; e < kDepth; ++e)
-        if (e * kSelBlock < ck) fetch(staged[e], e * kSelBlock);
-    float lmax = -INFINITY;
+            for (int w = 0; w < T::KW; ++w) acc[r][w] = 0.0f;
+        const bool has_keys = pass * T::kKeys + kg * T::KW * kSelBlock < ck;
+        for (int chunk = 0; chunk < chunks; ++chunk) {
+            __syncthreads();  // the previous chunk is consumed (and the query rows are staged)
 #pragma unroll
-    for (int e = 0; e < KPL; ++e) {
-        const int base = e * kSelBlock;
-        if (base < ck) {
-            const int rows = min(kSelBlock, ck - base);
-            __syncthreads();  // the previous block is consumed (and the query rows are staged)
-            store(staged[e % kDepth], base);
+            for (int i = 0; i < kSelStage; ++i) kblk[(srow + i * kRowStep) * T::kStride + scol] = staged[i];
             __syncthreads();
-            if (base + kDepth * kSelBlock < ck) fetch(staged[e % kDepth], base + kDepth * kSelBlock);
-            if (active && lane < rows && logit[e] > -INFINITY) {
-                const float* kr = kblk + lane * kstride;
-                float dot = 0.0f;
-                int d = 0;
-                // Batches of kSelBatch key values are read before their fma chain so the
-                // LDS reads of a batch are in flight together.
-                for (; d + kSelBatch <= dims; d += kSelBatch) {
-                    float kv[kSelBatch];
+            if (chunk + 1 < chunks) fetch(pass, chunk + 1);
+            else if ((pass + 1) * T::kKeys < ck) fetch(pass + 1, 0);
+            if (!has_keys) continue;
+            const float* kr = kblk + (kg * T::KW * kSelBlock + lane) * T::kStride;
+            const float* qr = qrows + r0 * qstride + chunk * T::kChan;
+            const int lim = min(T::kChan, dims - chunk * T::kChan);
+            auto quad = [&](int d) {
+                float kv[T::KW][4];
 #pragma unroll
-                    for (int i = 0; i < kSelBatch; ++i) kv[i] = kr[d + i];
+                for (int w = 0; w < T::KW; ++w)
 #pragma unroll
-                    for (int i = 0; i < kSelBatch; i += 4) {
-                        const float4 q4 = *reinterpret_cast<const float4*>(q + d + i);
-                        dot = fmaf(q4.x, kv[i], dot);
-                        dot = fmaf(q4.y, kv[i + 1], dot);
-                        dot = fmaf(q4.z, kv[i + 2], dot);
-                        dot = fmaf(q4.w, kv[i + 3], dot);
+                    for (int i = 0; i < 4; ++i) kv[w][i] = kr[w * kSelBlock * T::kStride + d + i];
+#pragma unroll
+                for (int r = 0; r < T::kRows; ++r) {
+                    const float4 q4 = *reinterpret_cast<const float4*>(qr + r * qstride + d);
+#pragma unroll
+                    for (int w = 0; w < T::KW; ++w) {
+                        acc[r][w] = fmaf(q4.x, kv[w][0], acc[r][w]);
+                        acc[r][w] = fmaf(q4.y, kv[w][1], acc[r][w]);
+                        acc[r][w] = fmaf(q4.z, kv[w][2], acc[r][w]);
+                        acc[r][w] = fmaf(q4.w, kv[w][3], acc[r][w]);
                     }
                 }
-                for (; d < dims; ++d) dot = fmaf(q[d], kr[d], dot);
-                logit[e] = dot * scale + logit[e];
+            };
+            int d = 0;
+            for (; d + 8 <= lim; d += 8) {
+                quad(d);
+                quad(d + 4);
             }
-            lmax = fmaxf(lmax, logit[e]);
+            for (; d + 4 <= lim; d += 4) quad(d);
+            for (; d < lim; ++d)
+#pragma unroll
+                for (int r = 0; r < T::kRows; ++r)
+#pragma unroll
+                    for (int w = 0; w < T::KW; ++w)
+                        acc[r][w] = fmaf(qr[r * qstride + d], kr[w * kSelBlock * T::kStride + d], acc[r][w]);
         }
+        if (pass + 1 == T::kPasses || (pass + 1) * T::kKeys >= ck) {
+            // The counts are requested only now: their latency overlaps the exchange, and the score
+            // phase keeps their registers.
+#pragma unroll
+            for (int e = 0; e < KPL; ++e) {
+                const int j = e * kSelBlock + lane;
+                const int w = kcount[min(j, ck - 1)];
+                kcnt[e] = j < ck ? max(0, w) : 0;
+            }
+        }
+        // To the row layout (the previous pass's dots are read before its first chunk barrier).
+        if (has_keys) {
+#pragma unroll
+            for (int r = 0; r < T::kRows; ++r)
+#pragma unroll
+                for (int w = 0; w < T::KW; ++w)
+                    dots[(r0 + r) * T::kKeys + (kg * T::KW + w) * kSelBlock + lane] = acc[r][w];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < T::kBlocks; ++e) prob[pass * T::kBlocks + e] = dots[wave * T::kKeys + e * kSelBlock + lane];
     }
     if (active) {
+        float lmax = -INFINITY;
 #pragma unroll
-        for (int m = 1; m < kWave; m <<= 1) lmax = fmaxf(lmax, __shfl_xor(lmax, m, kWave));
+        for (int e = 0; e < KPL; ++e) {
+            prob[e] = kcnt[e] > 0 ? prob[e] * scale + logf(static_cast<float>(kcnt[e])) : -INFINITY;
+            lmax = fmaxf(lmax, prob[e]);
+        }
+        lmax = wave_reduce_f32(lmax, [](float x, float y) { return fmaxf(x, y); });
         if (!(lmax > -INFINITY && lmax < INFINITY)) lmax = 0.0f;
         // Masses and their sum (lane partials in index order, then a fixed xor tree).
         float part = 0.0f;
 #pragma unroll
         for (int e = 0; e < KPL; ++e) {
             if (e * kSelBlock + lane < ck) {
-                logit[e] = expf(logit[e] - lmax);
-                part += logit[e];
+                prob[e] = expf(prob[e] - lmax);
+                part += prob[e];
             }
         }
-#pragma unroll
-        for (int m = 1; m < kWave; m <<= 1) part += __shfl_xor(part, m, kWave);
+        part = wave_reduce_f32(part, [](float x, float y) { return x + y; });
         const float denom = fmaxf(part, 1.17549435e-38f);
-        // Sort keys (~orderable(prob), j): ascending = descending probability, then index.
-        // Position i = KPL * lane + e initially holds key j = 64 e + lane.
-        uint64_t key[KPL];
 #pragma unroll
-        for (int e = 0; e < KPL; ++e) {
-            const int j = e * kSelBlock + lane;
-            key[e] = j < ck ? (static_cast<uint64_t>(~orderable(logit[e] / denom)) << 32) | static_cast<uint32_t>(j)
-                            : ~0ull;
-        }
-#pragma unroll
-        for (int kk = 2; kk <= kWave * KPL; kk <<= 1) {
-#pragma unroll
-            for (int jj = kk >> 1; jj > 0; jj >>= 1) {
-                if (jj >= KPL) {
-                    const int m = jj / KPL;
-                    const bool lower = (lane & m) == 0;
-#pragma unroll
-                    for (int e = 0; e < KPL; ++e) {
-                        const bool up = ((lane * KPL + e) & kk) == 0;
-                        const uint64_t other = shfl_xor_u64(key[e], m);
-                        // Keys are distinct (indices differ) except the equal padding keys.
-                        if ((key[e] < other) != (lower == up)) key[e] = other;
-                    }
-                } else {
-#pragma unroll
-                    for (int e = 0; e < KPL; ++e) {
-                        if ((e & jj) == 0) {
-                            const bool up = ((lane * KPL + e) & kk) == 0;
-                            const uint64_t x = key[e], y = key[e | jj];
-                            const bool swap = (x > y) == up;
-                            key[e] = swap ? y : x;
-                            key[e | jj] = swap ? x : y;
-                        }
-                    }
-                }
-            }
-        }
-        // Length of the kept prefix: every lane walks the same sequential double sum, one
-        // source lane (KPL sorted positions) per step, leaving the loop once per step.
-        const int floor_keep = max(1, minimum);
-        int kept = ck;
-        if (!(p >= 1.0f)) {
-            double run = 0.0;
-            for (int l = 0; l * KPL < ck; ++l) {
-                float prob[KPL];
-#pragma unroll
-                for (int e = 0; e < KPL; ++e)
-                    prob[e] = key_prob(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(key[e] >> 32), l)));
-                bool fail[KPL];
-#pragma unroll
-                for (int e = 0; e < KPL; ++e) {
-                    const int k = l * KPL + e;
-                    if (k < ck) run += static_cast<double>(prob[e]);
-                    const float before = static_cast<float>(run) - prob[e];
-                    fail[e] = k < ck && k >= floor_keep && !(before < p);
-                }
-                int first = ck;
-#pragma unroll
-                for (int e = KPL - 1; e >= 0; --e)
-                    if (fail[e]) first = l * KPL + e;
-                if (first < ck) {
-                    kept = first;
-                    break;
-                }
-            }
-        }
+        for (int e = 0; e < KPL; ++e) prob[e] = e * kSelBlock + lane < ck ? prob[e] / denom : -1.0f;
+        uint32_t keep = keep_prefix<KPL>(prob, ck, max(1, minimum), p, part < INFINITY);
         const bool qnonempty = qn[static_cast<int64_t>(b) * cq + c] > 0;
         int kept_rows = 0;  // key rows behind this row's kept clusters
 #pragma unroll
         for (int e = 0; e < KPL; ++e) {
-            const int k = lane * KPL + e;
-            if (k < ck) {
-                const int j = static_cast<int>(key[e] & 0xffffffffu);
-                const int n = kcount[j];
-                const bool on = k < kept && qnonempty && n > 0;
-                flags[j] = on;
-                kept_rows += on ? n : 0;
-            }
+            if (!qnonempty || kcnt[e] == 0) keep &= ~(1u << e);
+            kept_rows += keep & (1u << e) ? kcnt[e] : 0;
         }
         if (kept_keys) {
-#pragma unroll
-            for (int m = 1; m < kWave; m <<= 1) kept_rows += __shfl_xor(kept_rows, m, kWave);
+            kept_rows = wave_reduce_i32(kept_rows, [](int x, int y) { return x + y; });
             if (lane == 0)
                 kept_keys[static_cast<int64_t>(b) * re + c] = kept_rows + (extend ? valid_text : 0);  // as the map row
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         if (map) {
             uint8_t* mrow = map + (static_cast<int64_t>(b) * re + c) * ce;
-            for (int j = lane; j < ck; j += kWave) mrow[j] = flags[j];
+#pragma unroll
+            for (int e = 0; e < KPL; ++e) {
+                const int j = e * kSelBlock + lane;
+                if (j < ck) mrow[j] = (keep >> e) & 1u;
+            }
             if (extend && lane < 2) mrow[ck + lane] = lane == 0;  // video rows see valid text, never padding
         }
         if constexpr (kWork) {
             // Video rows keep their selected clusters and the valid text, never the padding.
-            int2* srow = work.segs + (static_cast<int64_t>(b) * re + c) * (ce + 2);
-            const int rk = write_segments(srow, kcnt, ck, ce, valid_text, text, sk,
-                                          [&](int j) { return j < ck ? flags[j] != 0 : j == ck; });
+            int2* segs = work.segs + (static_cast<int64_t>(b) * re + c) * (ce + 2);
+            const int rk = write_segments<KPL>(segs, kcnt, ck, ce, valid_text, text, sk,
+                                               [&](int j, int e) { return j < ck ? ((keep >> e) & 1u) != 0 : j == ck; });
             if (lane == 0)
                 __hip_atomic_store(work.row_keys + static_cast<int64_t>(b) * re + c, rk, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
@@ -376,9 +560,9 @@ __global__ __launch_bounds__(kSelWaves * kWave) void select_kernel(
             // The text rows: valid text sees every video key and the valid text, padding only
             // itself.
             const int r = cq + wave;
-            int2* srow = work.segs + (static_cast<int64_t>(b) * re + r) * (ce + 2);
-            const int rk = write_segments(srow, kcnt, ck, ce, valid_text, text, sk,
-                                          [&](int j) { return wave == 0 ? j < ck + 1 : j == ck + 1; });
+            int2* segs = work.segs + (static_cast<int64_t>(b) * re + r) * (ce + 2);
+            const int rk = write_segments<KPL>(segs, kcnt, ck, ce, valid_text, text, sk,
+                                               [&](int j, int) { return wave == 0 ? j < ck + 1 : j == ck + 1; });
             if (lane == 0)
                 __hip_atomic_store(work.row_keys + static_cast<int64_t>(b) * re + r, rk, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
@@ -430,19 +614,21 @@ __global__ __launch_bounds__(kSelWaves * kWave) void select_kernel(
     }
 }
 
-template <int KPL, bool kWide>
+template <int KPL>
 void launch_select(int blocks, size_t lds, hipStream_t stream, const float* qc, const float* kc, const int32_t* qn,
                    const int32_t* kn, int bh, int cq, int ck, int dims, float scale, float p, int minimum, int extend,
                    int valid_text, int text, uint8_t* map, int32_t* ext_q, int32_t* ext_k, int32_t* kept_keys,
                    int sq, int sk, const SelWork* work) {
+    const size_t qstride = (static_cast<size_t>(dims) + 3) & ~static_cast<size_t>(3);
+    lds = std::max(lds, sizeof(float) * (kSelWaves * qstride + SelTiles<KPL>::kLdsFloats));
     if (work)
-        hipLaunchKernelGGL((select_kernel<KPL, true, kWide>), dim3(static_cast<unsigned>(blocks)), dim3(kSelWaves * kWave),
-                           lds, stream, qc, kc, qn, kn, bh, cq, ck, dims, scale, p, minimum, extend, valid_text, text,
-                           map, ext_q, ext_k, kept_keys, sq, sk, *work);
+        hipLaunchKernelGGL((select_kernel<KPL, true>), dim3(static_cast<unsigned>(blocks)), dim3(kSelThreads), lds, stream,
+                           qc, kc, qn, kn, bh, cq, ck, dims, scale, p, minimum, extend, valid_text, text, map, ext_q,
+                           ext_k, kept_keys, sq, sk, *work);
     else
-        hipLaunchKernelGGL((select_kernel<KPL, false, kWide>), dim3(static_cast<unsigned>(blocks)), dim3(kSelWaves * kWave),
-                           lds, stream, qc, kc, qn, kn, bh, cq, ck, dims, scale, p, minimum, extend, valid_text, text,
-                           map, ext_q, ext_k, kept_keys, sq, sk, SelWork{});
+        hipLaunchKernelGGL((select_kernel<KPL, false>), dim3(static_cast<unsigned>(blocks)), dim3(kSelThreads), lds, stream,
+                           qc, kc, qn, kn, bh, cq, ck, dims, scale, p, minimum, extend, valid_text, text, map, ext_q,
+                           ext_k, kept_keys, sq, sk, SelWork{});
 }
 
 // Shared host entry: validation, LDS size and the launch over the per-lane key count.
@@ -455,26 +641,25 @@ int select_launch(const float* qc, const float* kc, const int32_t* q_counts, con
         return kInvalidValue;
     if (ck > kWave * 32) return kUnsupportedShape;
     const size_t qstride = (static_cast<size_t>(dims) + 3) & ~static_cast<size_t>(3);
-    size_t lds = sizeof(float) * (kSelWaves * qstride + static_cast<size_t>(kSelBlock) * (dims + 1)) +
-                 static_cast<size_t>(kSelWaves) * ck;
+    // Shapes this entry has always refused stay refused (a key block of 64 rows and a flag byte per
+    // row and key beside the query rows); the kernel itself needs at most 60 KB for those it takes.
+    if (sizeof(float) * (kSelWaves * qstride + static_cast<size_t>(kSelBlock) * (dims + 1)) +
+            static_cast<size_t>(kSelWaves) * ck > 64 * 1024)
+        return kUnsupportedShape;
+    size_t lds = 0;
     if (work) {
         // The last workgroup of an entry reuses the LDS for its query offsets, row lengths and sort keys.
         const size_t re = static_cast<size_t>(extend ? cq + 2 : cq);
-        lds = std::max(lds, sizeof(int) * (2 * re + 2) + sizeof(uint64_t) * kSortCap);
+        lds = sizeof(int) * (2 * re + 2) + sizeof(uint64_t) * kSortCap;
+        if (lds > 64 * 1024) return kUnsupportedShape;
     }
-    if (lds > 64 * 1024) return kUnsupportedShape;
     const int blocks = bh * static_cast<int>(ceil_div(cq, kSelWaves));
     const float scale = static_cast<float>(std::pow(static_cast<double>(dims), -0.5));
     auto* s = static_cast<hipStream_t>(stream);
     const int per_lane = static_cast<int>(ceil_div(ck, kWave));
-#define PECO_SELECT_W(K, W)                                                                                     \
-    launch_select<K, W>(blocks, lds, s, qc, kc, q_counts, k_counts, bh, cq, ck, dims, scale, p, minimum, extend, \
-                        valid_text, text, map, ext_q, ext_k, kept_keys, sq, sk, work)
-#define PECO_SELECT(K)                                                                                          \
-    do {                                                                                                        \
-        if (dims <= 128) PECO_SELECT_W(K, false);                                                               \
-        else PECO_SELECT_W(K, true);                                                                            \
-    } while (0)
+#define PECO_SELECT(K)                                                                                             \
+    launch_select<K>(blocks, lds, s, qc, kc, q_counts, k_counts, bh, cq, ck, dims, scale, p, minimum, extend, valid_text, \
+                     text, map, ext_q, ext_k, kept_keys, sq, sk, work)
     if (per_lane <= 1) PECO_SELECT(1);
     else if (per_lane <= 2) PECO_SELECT(2);
     else if (per_lane <= 4) PECO_SELECT(4);
@@ -482,7 +667,6 @@ int select_launch(const float* qc, const float* kc, const int32_t* q_counts, con
     else if (per_lane <= 16) PECO_SELECT(16);
     else PECO_SELECT(32);
 #undef PECO_SELECT
-#undef PECO_SELECT_W
     return hipGetLastError();
 }
 

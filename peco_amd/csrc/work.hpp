@@ -83,13 +83,22 @@ __host__ __device__ inline SelWork sel_work_layout(int32_t* base, int bh, int sq
     return w;
 }
 
+// DPP move of v by control `kCtrl`, 0 where the source lane is outside the row or row_mask leaves
+// the row out.
+template <int kCtrl, int kRowMask = 0xf> __device__ __forceinline__ int dpp_or_zero(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, kCtrl, kRowMask, 0xf, false);
+}
+
+// Inclusive scan over a wavefront: four shifts inside the 16-lane rows, then the row sums
+// broadcast to the rows after them. All of it is VALU work (about a tenth of the latency of six
+// ds_bpermute round trips).
 __device__ __forceinline__ int wave_incl_scan(int v) {
-    const int lane = lane_id();
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-        const int y = __shfl_up(v, d, kWave);
-        if (lane >= d) v += y;
-    }
+    v += dpp_or_zero<0x111>(v);       // row_shr:1
+    v += dpp_or_zero<0x112>(v);       // row_shr:2
+    v += dpp_or_zero<0x114>(v);       // row_shr:4
+    v += dpp_or_zero<0x118>(v);       // row_shr:8
+    v += dpp_or_zero<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+    v += dpp_or_zero<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
     return v;
 }
 
