@@ -248,6 +248,16 @@ int peco_base_offset_attention(const void* q, const int32_t* out_index, const fl
                                size_t workspace_ints, int bh, int sq, int sk, int oi_rows, int d, int cq, int ck,
                                int dtype, void* stream);
 
+/* Projected rows into a head-major attention buffer (peco/processor.py:159-190 after the projection
+ * and norm): input [batch, heads, rows, dims] (fp16/bf16, dims 64 or 128, element strides of
+ * batch, head and row, channels adjacent, rows 16-byte aligned) is written to rows [first, first +
+ * rows) of output [batch, heads, length, dims]. With cos/sin (fp32 [rows, dims], both or neither)
+ * the rows are rotated over interleaved channel pairs: x * cos + (-x1, x0) * sin in fp32, rounded
+ * once to the dtype. */
+int peco_place_heads(const void* input, int64_t stride_batch, int64_t stride_head, int64_t stride_row, void* output,
+                     const float* cos, const float* sin, int batch, int heads, int rows, int first, int length,
+                     int dims, int dtype, void* stream);
+
 /* peco_sparse_attention without a workspace argument. No counterpart in the reference: it is
  * for callers that cannot allocate device memory (code under HIP graph capture, serving loops
  * that forbid hipMalloc). The work list lives in a static per-device array of 1048576 int32

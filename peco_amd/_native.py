@@ -131,6 +131,7 @@ SIGNATURES = {
     "peco_select_work_size": (Z, [I] * 5),
     "peco_select_work": (I, [P] * 4 + [I] * 4 + [ctypes.c_float] + [I] * 6 + [P] * 4 + [Z, P]),
     "peco_sparse_attention_work": (I, [P] * 5 + [I, P, P, I, I, P, Z] + [I] * 7 + [P]),
+    "peco_place_heads": (I, [P] + [ctypes.c_int64] * 3 + [P] * 3 + [I] * 7 + [P]),
     "peco_base_offset_attention": (I, [P, P, P, I] + [P] * 9 + [I, I] + [P] * 5 + [Z] + [I] * 8 + [P]),
 }
 
@@ -181,6 +182,21 @@ def current_stream(device, *tensors) -> ctypes.c_void_p:
         if t is not None:
             t.record_stream(stream)
     return ctypes.c_void_p(stream.cuda_stream)
+
+
+def plain_tensors(*tensors) -> bool:
+    """True when raw pointers may stand for these tensors in place of torch operations: ordinary
+    tensors, not under tracing or a functorch transform, without a forward-mode tangent."""
+    import torch
+
+    if torch.compiler.is_compiling():
+        return False
+    for t in tensors:
+        if type(t) not in (torch.Tensor, torch.nn.Parameter) or torch._C._functorch.is_functorch_wrapped_tensor(t):
+            return False
+        if torch.autograd.forward_ad.unpack_dual(t).tangent is not None:
+            return False
+    return True
 
 
 # hipEventDisableSystemFence (hip_runtime_api.h): the event skips the system-scope cache writeback

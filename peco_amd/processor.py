@@ -22,7 +22,7 @@ import torch
 import torch.nn.functional as F
 from torch.nn.attention import SDPBackend, sdpa_kernel
 
-from . import clustering_cuda
+from . import _native, clustering_cuda
 from .attention_cuda import base_offset_attention, sparse_attention, sparse_attention_work
 from .quantization import _validate_bits
 
@@ -116,6 +116,42 @@ def _apply_rotary_emb(x, freqs_cis):
     real, imag = x.reshape(*x.shape[:-1], -1, 2).unbind(-1)
     rotated = torch.stack([-imag, real], dim=-1).flatten(3)
     return (x.float() * cos + rotated.float() * sin).to(x.dtype)
+
+
+def _per_channel_norm(norm):
+    """True for a norm module that acts on the last axis alone, whatever the axes before it, with
+    nothing attached that could see the shape it is called with."""
+    hooks = torch.nn.modules.module
+    return type(norm) in (torch.nn.RMSNorm, torch.nn.LayerNorm) and len(norm.normalized_shape) == 1 and \
+        "forward" not in vars(norm) and not norm._forward_hooks and not norm._forward_pre_hooks and \
+        not hooks._global_forward_hooks and not hooks._global_forward_pre_hooks
+
+
+def _published_rotary(fn):
+    return fn is _apply_rotary_emb or (getattr(fn, "__module__", "") == "diffusers.models.embeddings" and
+                                       getattr(fn, "__name__", "") == "apply_rotary_emb")
+
+
+def _rotary_tables(fn, freqs, rows, dim, device):
+    """(cos, sin) when the rotary embedding is the published one over plain fp32 [rows, dim] tables
+    that the placing kernel can read, else None."""
+    if not _published_rotary(fn) or not isinstance(freqs, (tuple, list)) or len(freqs) != 2 or \
+            not all(isinstance(t, torch.Tensor) for t in freqs) or not _native.plain_tensors(*freqs):
+        return None
+    for t in freqs:
+        if t.dtype != torch.float32 or t.shape != (rows, dim) or t.device != device or not t.is_contiguous() or \
+                t.data_ptr() % 16:
+            return None
+    return tuple(freqs)
+
+
+def _placeable(part, buffer):
+    """Whether place_heads takes ``part`` [B, H, rows, D] into ``buffer`` [3, B, H, S, D]: the shapes
+    and dtype agree and its rows start on 16 bytes with adjacent channels."""
+    return part.shape[:2] == buffer.shape[1:3] and part.shape[3] == buffer.shape[4] and part.shape[3] in (64, 128) and \
+        part.shape[2] > 0 and part.dtype == buffer.dtype and part.dtype in (torch.bfloat16, torch.float16) and \
+        part.is_cuda and part.stride(3) == 1 and all(s % 8 == 0 for s in part.stride()[:3]) and \
+        part.data_ptr() % 16 == 0 and part.shape[0] <= 65535 and _native.plain_tensors(part, buffer)
 
 
 class _FitResult:
@@ -300,9 +336,10 @@ class PecoAttention:
 
         ``attention_mask`` is ignored: which text rows are valid comes from the shared
         InferenceContext. The sequence is [video rows, text rows]. Each projection of each
-        part is written once, head-major, into its slot of one [3, B, H, S, D] buffer (the
-        copy that splits the heads also places the rows), so no concatenation copies are
-        made. Video rows get the rotary embedding; text rows never do. Double-stream blocks
+        part is written once, head-major, into its slot of one [3, B, H, S, D] buffer, so no
+        concatenation copies are made; one launch per projection splits the heads, applies the
+        rotary embedding and places the rows (torch operations do it for tensors that launch does
+        not take). Video rows get the rotary embedding; text rows never do. Double-stream blocks
         (``add_q_proj`` set) project the text with their added projections and norms,
         single-stream blocks with the same ones as the video.
         """
@@ -324,15 +361,23 @@ class PecoAttention:
             rows = source.shape[1]
             for slot, proj in enumerate(projections):
                 part = proj(source).unflatten(2, (attn.heads, -1)).transpose(1, 2)  # [B, H, rows, D] view
+                tables = None
                 if slot < 2:
                     if norms[slot] is not None:
-                        part = norms[slot](part)
+                        # The rows as projected, where the norm cannot tell: no copy into head order first.
+                        swap = part.is_cuda and _per_channel_norm(norms[slot])
+                        part = norms[slot](part.transpose(1, 2)).transpose(1, 2) if swap else norms[slot](part)
                     if freqs is not None:
-                        part = rotary(part, freqs)
+                        tables = _rotary_tables(rotary, freqs, rows, part.shape[3], part.device)
+                        if tables is None:
+                            part = rotary(part, freqs)
                 if qkv is None:
                     batch, heads, _, dim = part.shape
                     qkv = torch.empty((3, batch, heads, length, dim), dtype=part.dtype, device=part.device)
-                qkv[slot, :, :, first:first + rows] = part
+                if _placeable(part, qkv):
+                    clustering_cuda.place_heads(part, qkv[slot], first, tables)
+                else:
+                    qkv[slot, :, :, first:first + rows] = part if tables is None else rotary(part, freqs)
             first += rows
         output = self.attention(qkv[0], qkv[1], qkv[2]).transpose(1, 2)  # [B, S, H, D] view
         video = hidden_states.shape[1]

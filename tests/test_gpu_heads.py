@@ -1,0 +1,72 @@
+"""The processor prologue's placing kernel (heads.hip) against the torch expression it stands for,
+bit for bit, and the processor call with it against the call that takes the torch path."""
+import pytest
+import torch
+
+from peco_amd import clustering_cuda, processor
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _tables(rows, dim, g):
+    theta = torch.rand(rows, dim // 2, generator=g) * 6.3
+    return tuple(t.repeat_interleave(2, -1).to(DEV).contiguous() for t in (theta.cos(), theta.sin()))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("batch,heads,rows,first,length", [
+    (1, 1, 1, 0, 1), (1, 7, 15, 3, 20), (2, 8, 16, 0, 16), (1, 9, 17, 5, 40), (1, 24, 333, 0, 400), (3, 2, 33, 7, 40)])
+def test_place_heads_matches_torch(dtype, dim, batch, heads, rows, first, length):
+    g = torch.Generator().manual_seed(rows * heads + dim)
+    x = torch.randn(batch, rows, heads, dim, generator=g).to(dtype).to(DEV)
+    x[0, 0, 0, :2] = torch.tensor([float("inf"), -0.0], dtype=dtype)
+    wide = torch.zeros(batch, rows, heads, dim + 8, dtype=dtype, device=DEV)  # rows with a gap between heads
+    wide[..., :dim] = x
+    tables = _tables(rows, dim, g)
+    for part in (x.transpose(1, 2), x.transpose(1, 2).contiguous(), wide[..., :dim].transpose(1, 2)):
+        for rotary in (None, tables):
+            out = torch.full((batch, heads, length, dim), 7.0, dtype=dtype, device=DEV)
+            ref = out.clone()
+            clustering_cuda.place_heads(part, out, first, rotary)
+            ref[:, :, first:first + rows] = part if rotary is None else processor._apply_rotary_emb(part, rotary)
+            assert torch.equal(torch.isnan(out), torch.isnan(ref))
+            assert torch.equal(out.nan_to_num(3.0), ref.nan_to_num(3.0))
+
+
+class _Block(torch.nn.Module):
+    def __init__(self, heads, dim, double):
+        super().__init__()
+        width = heads * dim
+        self.heads = heads
+        linear = lambda: torch.nn.Linear(width, width)  # noqa: E731
+        self.to_q, self.to_k, self.to_v = linear(), linear(), linear()
+        self.norm_q, self.norm_k = torch.nn.RMSNorm(dim, eps=1e-6), torch.nn.RMSNorm(dim, eps=1e-6)
+        self.add_q_proj = None
+        if double:
+            self.add_q_proj, self.add_k_proj, self.add_v_proj = linear(), linear(), linear()
+            self.norm_added_q, self.norm_added_k = torch.nn.LayerNorm(dim), None
+
+
+@pytest.mark.parametrize("double", [False, True])
+@pytest.mark.parametrize("text", [0, 40])
+def test_call_matches_the_torch_prologue(double, text, monkeypatch):
+    heads, dim, video = 3, 64, 500
+    torch.manual_seed(5)
+    block = _Block(heads, dim, double).to(DEV, torch.bfloat16)
+    g = torch.Generator().manual_seed(9)
+    hidden = torch.randn(1, video, heads * dim, generator=g).to(DEV, torch.bfloat16)
+    enc = torch.randn(1, text, heads * dim, generator=g).to(DEV, torch.bfloat16) if text else None
+    freqs = _tables(video, dim, g)
+    layer = processor.PecoAttention(0, processor.PecoConfig(), processor.InferenceContext(5, text, text))
+    layer.attention = lambda q, k, v: torch.cat((q, k, v), -1)
+    got = layer(block, hidden, enc, image_rotary_emb=freqs)
+    # A rotary function of the caller's own, and norms with a hook, take the torch operations.
+    monkeypatch.setattr(processor, "_rotary_function", lambda: lambda x, f: processor._apply_rotary_emb(x, f))
+    monkeypatch.setattr(processor, "_placeable", lambda part, buffer: False)
+    for norm in (block.norm_q, block.norm_k):
+        norm.register_forward_hook(lambda module, args, out: None)
+    ref = layer(block, hidden, enc, image_rotary_emb=freqs)
+    assert torch.equal(got[0], ref[0])
+    assert (got[1] is None and ref[1] is None) if not text else torch.equal(got[1], ref[1])
