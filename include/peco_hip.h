@@ -248,6 +248,14 @@ int peco_base_offset_attention(const void* q, const int32_t* out_index, const fl
                                size_t workspace_ints, int bh, int sq, int sk, int oi_rows, int d, int cq, int ck,
                                int dtype, void* stream);
 
+/* Dense attention of a warm-up step (peco/processor.py:52-65) on the sparse kernel's MFMA path: of
+ * q/k/v [bh, s, d] (fp16/bf16, d 64 or 128), rows [0, valid) attend to each other and so do rows
+ * [valid, s). workspace: peco_dense_attention_workspace_size int32 (8-byte aligned, need not be
+ * cleared). */
+size_t peco_dense_attention_workspace_size(int bh, int s);
+int peco_dense_attention(const void* q, const void* k, const void* v, void* output, int valid, int32_t* workspace,
+                         size_t workspace_ints, int bh, int s, int d, int dtype, void* stream);
+
 /* Projected rows into a head-major attention buffer (peco/processor.py:159-190 after the projection
  * and norm): input [batch, heads, rows, dims] (fp16/bf16, dims 64 or 128, element strides of
  * batch, head and row, channels adjacent, rows 16-byte aligned) is written to rows [first, first +

@@ -258,6 +258,38 @@ def sparse_attention_work(
     return output
 
 
+def dense_supported(q, k, v, valid_length) -> bool:
+    """Whether ``dense_attention`` takes these tensors (anything else is the caller's to run)."""
+    return isinstance(valid_length, int) and all(isinstance(t, torch.Tensor) for t in (q, k, v)) and q.ndim == 4 and \
+        q.shape == k.shape == v.shape and 0 <= valid_length <= q.shape[2] and q.shape[3] in (64, 128) and \
+        1 <= q.shape[0] * q.shape[1] <= 65535 and q.dtype in (torch.float16, torch.bfloat16) and \
+        q.dtype == k.dtype == v.dtype and q.is_cuda and q.device == k.device == v.device and \
+        not (torch.is_grad_enabled() and any(t.requires_grad for t in (q, k, v))) and \
+        not torch.is_autocast_enabled("cuda") and _native.plain_tensors(q, k, v) and _device_is_gfx950(q.device)
+
+
+def dense_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, valid_length: int) -> torch.Tensor:
+    """Dense attention over rows [0, valid_length) and over the rows after them separately
+    (peco/processor.py:52-65) on the sparse kernel, for tensors ``dense_supported`` accepts; the
+    result has the strides of ``empty_like(q)``."""
+    like = q
+    q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+    batch, heads, length, dim = q.shape
+    output = torch.empty_like(q)
+    with torch.cuda.device(q.device):
+        library = _native.library()
+        ints = library.peco_dense_attention_workspace_size(batch * heads, length)
+        workspace = torch.empty(max(ints, 1), dtype=torch.int32, device=q.device)
+        error = library.peco_dense_attention(
+            _native.ptr(q), _native.ptr(k), _native.ptr(v), _native.ptr(output), valid_length, _native.ptr(workspace),
+            ints, batch * heads, length, dim, 0 if q.dtype == torch.float16 else 1,
+            _native.current_stream(q.device, q, k, v, output, workspace))
+        if error:
+            message = library.peco_attention_error_string(error).decode("utf-8", errors="replace")
+            raise RuntimeError(f"PECO HIP dense attention launch failed: {message} ({error})")
+    return output if like.is_contiguous() else torch.empty_like(like).copy_(output)
+
+
 def centroid_planes(centroids: torch.Tensor):
     """Key centroids [BH, K, D] fp32 as three int8 planes and a scale per centroid:
     C = cs * (P0 + P1/128 + P2/16384) to within 2^-21 * max|C| of each centroid (the last

@@ -266,8 +266,8 @@ template <int D> struct Tiles {
 
 // Issue the direct-to-LDS loads of one K and one V tile (no wait), or the share of a wave
 // that is one of NL loaders (rank `first`): the tile's 4*kLoads spans of 64 lanes x 16 bytes
-// per tensor go round-robin to the loaders. Rows past the stream end read row 0 of the head:
-// their K scores are masked to -inf and their P is 0.
+// per tensor go round-robin to the loaders. Rows past the stream end repeat its last row: their K
+// scores are masked to -inf and their P is 0.
 template <int D, int NL>
 __device__ __forceinline__ void load_tile_lds(uint16_t* ks, uint16_t* vs, const uint16_t* kh, const uint16_t* vh,
                                               const int* prow, int first, int lane) {
@@ -331,14 +331,12 @@ __device__ __forceinline__ void attention_item(
     const int32_t* __restrict__ counts, const int32_t* __restrict__ items, int cap, uint16_t* __restrict__ out,
     const int32_t* __restrict__ out_index, int oi_rows, const int32_t* __restrict__ k_index,
     const float* __restrict__ qcent, int qcent_rows, float levels, int bhn, int band, int sq, int sk, int cq,
-    int ck, float scale_log2) {
+    int ck, float scale_log2, float lazy) {
     constexpr bool kIndexedKV = kMode == kIndexed || kMode == kIndexedQuantQ;
     constexpr bool kQuantLoad = kMode == kQuantQ || kMode == kIndexedQuantQ;
     using T = Tiles<D>;
     constexpr int S = D / 16;       // k-steps of S^T over channels
     constexpr int NB = D / 32;      // 32-channel blocks of O^T
-    // Scores may run up to 2^8 above the running maximum before O is rescaled.
-    constexpr float kLazyLog2 = 8.0f;
     // K tiles (buffers 0, 1) and V tiles (2, 3) in one array: after the last tile the paired
     // waves exchange their softmax states through it, which takes more than the K half.
     constexpr int NT = kWaves * kWave;           // threads of the workgroup
@@ -488,8 +486,11 @@ __device__ __forceinline__ void attention_item(
     const int32_t* kidx = kIndexedKV ? k_index + head * oi_rows : nullptr;
     const int prow_entry = kRowsPerWave * wave + lane % kRowsPerWave;
     const bool prow_owner = lane < kRowsPerWave;
-    // Stream position (cluster-order row) of stream row r; rows past the stream read row 0.
-    auto stream_pos = [&](int r) { return r < L ? static_cast<int>(min(static_cast<uint32_t>(row_of(r)), sk_last)) : 0; };
+    // Stream position (cluster-order row) of stream row r; rows past the stream repeat its last row
+    // (their scores are masked; a row of the stream itself, so that no value the item's queries do
+    // not attend to is ever multiplied in).
+    const int l_last = max(L - 1, 0);
+    auto stream_pos = [&](int r) { return static_cast<int>(min(static_cast<uint32_t>(row_of(min(r, l_last))), sk_last)); };
     // Physical row of stream position p, given k_index[p] (clamped to the head's rows, so a bad
     // permutation cannot read out of bounds).
     auto physical = [&](int p, int raw) {
@@ -515,7 +516,6 @@ __device__ __forceinline__ void attention_item(
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) oacc[nb] = f32x16{};
     float m_run = -INFINITY, l_run = 0.0f, neg_m = 0.0f;
-    const float lazy = kLazyLog2 / scale_log2;
 
     const uint16_t* kh = k + head * sk * D;
     const uint16_t* vh = v + head * sk * D;
@@ -811,11 +811,11 @@ __global__ __launch_bounds__(kWaves * kWave, 8 / kWaves) void sparse_attention_k
     const int32_t* __restrict__ counts, const int32_t* __restrict__ items, int cap, uint16_t* __restrict__ out,
     const int32_t* __restrict__ out_index, int oi_rows, const int32_t* __restrict__ k_index,
     const float* __restrict__ qcent, int qcent_rows, float levels, int bhn, int band, int sq, int sk, int cq,
-    int ck, float scale_log2, int32_t* __restrict__ queues, int nwg) {
+    int ck, float scale_log2, float lazy, int32_t* __restrict__ queues, int nwg) {
     if constexpr (!kPersist) {
         attention_item<DT, D, kMode, kWaves>(blockIdx.x, q, k, v, selected, kprefix, segs, counts, items, cap, out,
                                              out_index, oi_rows, k_index, qcent, qcent_rows, levels, bhn, band, sq,
-                                             sk, cq, ck, scale_log2);
+                                             sk, cq, ck, scale_log2, lazy);
     } else {
         __shared__ int next;
         const int total = cap * bhn;
@@ -832,7 +832,7 @@ __global__ __launch_bounds__(kWaves * kWave, 8 / kWaves) void sparse_attention_k
             x = g % kItemQueues;
             attention_item<DT, D, kMode, kWaves>(g, q, k, v, selected, kprefix, segs, counts, items, cap, out,
                                                  out_index, oi_rows, k_index, qcent, qcent_rows, levels, bhn, band, sq,
-                                                 sk, cq, ck, scale_log2);
+                                                 sk, cq, ck, scale_log2, lazy);
         }
         if (threadIdx.x == 0 && atomicAdd(&queues[kItemQueues], 1) == nwg - 1) {
             for (int x = 0; x <= kItemQueues; ++x)
@@ -1330,20 +1330,26 @@ int attention_head_band(int bh, int sk, int d) {
 // sparse_attention_kernel (two resident workgroups per CU take items from the queues): 544p
 // attention 5.4% and 720p 4.2% faster than one workgroup per item, while at 480p (5.6 slots
 // per workgroup, items of about 100 us) taking each item costs more than it saves (+2.3%).
+// lazy_log2: scores may run up to 2^lazy_log2 above the running maximum before O is rescaled. The
+// sparse calls use kLazyLog2 (rescaling at every new maximum costs a few percent); 0 keeps the
+// largest weight of a row at exactly 1 when P is rounded to 16 bits, as an exact softmax does.
+constexpr float kLazyLog2 = 8.0f;
 constexpr int kPersistItems = 8;
 int launch_attention_kernel(const void* q, const void* k, const void* v, const uint8_t* selected,
                             const int32_t* kprefix, const int2* segs, const int32_t* counts, const int32_t* items,
                             int cap, void* output, const int32_t* out_index, int out_index_rows,
                             const int32_t* k_index, const float* q_centroids, int q_clusters, int bits, int bh,
-                            int sq, int sk, int d, int cq, int ck, int dtype, int32_t* queues, hipStream_t s) {
+                            int sq, int sk, int d, int cq, int ck, int dtype, int32_t* queues, int item_rows,
+                            float lazy_log2, hipStream_t s) {
     const int mode = k_index ? (q_centroids ? kIndexedQuantQ : kIndexed) : (q_centroids ? kQuantQ : kPacked);
     const float levels = static_cast<float>((1 << bits) - 1);
     const size_t lds_attn = sizeof(int) * 2 * (static_cast<size_t>(ck) + 1);
     const float scale_log2 = static_cast<float>(1.4426950408889634 / std::sqrt(static_cast<double>(d)));
+    const float lazy = lazy_log2 / scale_log2;  // in units of the raw scores
     const int64_t total = static_cast<int64_t>(cap) * bh;
-    // Items of 2 * kQTile rows (attention_item_rows, the builders' rule) run on 8-wavefront
+    // Items of 2 * kQTile rows (item_rows, as the work list was cut) run on 8-wavefront
     // workgroups, one per CU; others on 4-wavefront ones, two per CU.
-    const int waves = attention_item_rows(sq) == 2 * kQTile ? 8 : 4;
+    const int waves = item_rows == 2 * kQTile ? 8 : 4;
     const int nwg = static_cast<int>(
         std::min<int64_t>(total, (8 / waves) * static_cast<int64_t>(device_compute_units())));
     if (queues && total < static_cast<int64_t>(kPersistItems) * nwg) queues = nullptr;
@@ -1356,7 +1362,7 @@ int launch_attention_kernel(const void* q, const void* k, const void* v, const u
 #define PECO_ATTN_P(DT_, D_, M_, P_, W_)                                                                           \
     hipLaunchKernelGGL((sparse_attention_kernel<DT_, D_, M_, P_, W_>), grid, dim3(W_ * kWave), lds_attn, s, qp, kp, \
                        vp, selected, kprefix, segs, counts, items, cap, op, out_index, out_index_rows, k_index,      \
-                       q_centroids, q_clusters, levels, bh, band, sq, sk, cq, ck, scale_log2, queues, nwg)
+                       q_centroids, q_clusters, levels, bh, band, sq, sk, cq, ck, scale_log2, lazy, queues, nwg)
 #define PECO_ATTN(DT_, D_, M_, W_)                                                                                 \
     do {                                                                                                           \
         if (queues) PECO_ATTN_P(DT_, D_, M_, true, W_);                                                            \
@@ -1415,7 +1421,8 @@ int launch_sparse_attention(const void* q, const void* k, const void* v, const u
                            nullptr, workspace, bh, sq, sk, cq, ck, attention_item_rows(sq));
     const WorkLayout W = work_layout(workspace, bh, sq, cq, ck);
     return launch_attention_kernel(q, k, v, selected, W.kprefix, nullptr, W.counts, W.items, W.cap, output, out_index,
-                                   out_index_rows, k_index, nullptr, 0, 0, bh, sq, sk, d, cq, ck, dtype, nullptr, s);
+                                   out_index_rows, k_index, nullptr, 0, 0, bh, sq, sk, d, cq, ck, dtype, nullptr,
+                                   attention_item_rows(sq), kLazyLog2, s);
 }
 
 }  // namespace
@@ -1476,7 +1483,73 @@ PECO_API int peco_sparse_attention_work(const void* q, const void* k, const void
     return launch_attention_kernel(q, k, v, nullptr, nullptr, W.segs, W.counts, W.items, W.cap, output, out_index,
                                    out_index_rows, k_index, q_centroids, q_centroids ? q_clusters : 0,
                                    q_centroids ? bits : 0, bh, sq, sk, d, cq, ck, dtype, W.queues,
-                                   static_cast<hipStream_t>(stream));
+                                   attention_item_rows(sq), kLazyLog2, static_cast<hipStream_t>(stream));
+}
+
+// Dense attention of a warm-up step (peco/processor.py:52-65): rows [0, valid) attend to each other
+// and so do rows [valid, s), as two row groups of the work list above. MFMA-bound: full items over
+// one long key segment. Library SDPA, which needs each segment sliced into contiguous copies, took
+// 21.9 ms for 24 heads x 32896 rows x 128 channels in bf16 (609 TFLOP/s) and 1.64 ms at 7006 rows;
+// here 12.5 ms (1067 TFLOP/s; large bf16 matrix products reach 1190-1250 on this card) and 0.71
+// ms. O is rescaled at every new row maximum (see lazy_log2): with the sparse calls' lazy
+// threshold the error against 64 bits was 10% above SDPA's on peaked rows.
+namespace peco {
+namespace {
+
+// Work list of the two groups, one workgroup per head: per group one key segment, items of `tile`
+// rows in row order (all of a group cost alike, the valid rows' group first), zeroed queues.
+__global__ __launch_bounds__(256) void build_dense_kernel(int32_t* ws, int bhn, int s, int valid, int tile) {
+    const SelWork W = sel_work_layout(ws, bhn, s, 2, 2);
+    const int bh = blockIdx.x, tid = threadIdx.x;
+    const int n0 = static_cast<int>(ceil_div(valid, tile)), n1 = static_cast<int>(ceil_div(s - valid, tile));
+    int32_t* items = W.items + static_cast<int64_t>(bh) * W.cap * 3;
+    for (int i = tid; i < n0 + n1; i += blockDim.x) {
+        const int g = i >= n0;
+        const int begin = (g ? valid : 0) + (g ? i - n0 : i) * tile;
+        items[3 * i + 0] = begin;
+        items[3 * i + 1] = g;
+        items[3 * i + 2] = min(tile, (g ? s : valid) - begin);
+    }
+    if (tid < 2) {
+        const int rows = tid ? s - valid : valid;
+        int2* seg = W.segs + (static_cast<int64_t>(bh) * 2 + tid) * 4;
+        seg[0] = int2{rows > 0 ? 1 : 0, rows};
+        seg[1] = rows > 0 ? int2{tid ? valid : 0, 0} : int2{0, 0x7fffffff};
+        seg[2] = int2{0, 0x7fffffff};
+    }
+    if (tid == 0) W.counts[bh] = n0 + n1;
+    if (bh == 0 && tid < kQueueInts) W.queues[tid] = 0;
+}
+
+// Rows per item: full 256-row items on 8-wavefront workgroups when they still fill the CUs twice
+// (every K/V tile then serves twice the rows: 11.8 against 12.3 ms at 24 heads x 32896 rows, 0.62
+// against 0.63 ms at 7006), else 128-row items, which spread a short call over more CUs.
+int dense_item_rows(int bh, int s) {
+    return static_cast<int64_t>(bh) * (s / (2 * kQTile)) >= 2 * static_cast<int64_t>(device_compute_units()) ? 2 * kQTile
+                                                                                                           : kQTile;
+}
+
+}  // namespace
+}  // namespace peco
+
+PECO_API size_t peco_dense_attention_workspace_size(int bh, int s) {
+    if (bh < 1 || s < 0) return 0;
+    return sel_work_ints(bh, s, 2, 2);
+}
+
+PECO_API int peco_dense_attention(const void* q, const void* k, const void* v, void* output, int valid, int32_t* workspace,
+                                  size_t workspace_ints, int bh, int s, int d, int dtype, void* stream) {
+    if (!q || !k || !v || !output || !workspace || bh < 1 || bh > 65535 || s < 0 || valid < 0 || valid > s ||
+        (d != 64 && d != 128) || (dtype != kF16 && dtype != kBF16))
+        return kInvalidValue;
+    if (s == 0) return kOk;
+    if (workspace_ints < sel_work_ints(bh, s, 2, 2)) return kWorkspaceTooSmall;
+    const auto st = static_cast<hipStream_t>(stream);
+    const int tile = dense_item_rows(bh, s);
+    hipLaunchKernelGGL(build_dense_kernel, dim3(bh), dim3(256), 0, st, workspace, bh, s, valid, tile);
+    const SelWork W = sel_work_layout(workspace, bh, s, 2, 2);
+    return launch_attention_kernel(q, k, v, nullptr, nullptr, W.segs, W.counts, W.items, W.cap, output, nullptr, 0,
+                                   nullptr, nullptr, 0, 0, bh, s, s, d, 2, 2, dtype, W.queues, tile, 0.0f, st);
 }
 
 // Base-Offset integer-score attention (an extension with no counterpart in the reference; see

@@ -23,7 +23,8 @@ import torch.nn.functional as F
 from torch.nn.attention import SDPBackend, sdpa_kernel
 
 from . import _native, clustering_cuda
-from .attention_cuda import base_offset_attention, sparse_attention, sparse_attention_work
+from .attention_cuda import base_offset_attention, dense_supported, sparse_attention, sparse_attention_work
+from .attention_cuda import dense_attention as dense_attention_hip
 from .quantization import _validate_bits
 
 
@@ -61,7 +62,10 @@ class InferenceContext:
 
 
 def dense_attention(query, key, value, valid_length):
-    """Dense SDPA over [0, valid_length) and the padding segment separately (peco/processor.py:52-65)."""
+    """Dense attention over [0, valid_length) and the padding segment separately (peco/processor.py:52-65):
+    on the sparse kernel's MFMA path for the 16-bit tensors it takes in inference, else SDPA."""
+    if dense_supported(query, key, value, valid_length):
+        return dense_attention_hip(query, key, value, valid_length)
     output = torch.empty_like(query)
     backend = [SDPBackend.FLASH_ATTENTION, SDPBackend.EFFICIENT_ATTENTION, SDPBackend.MATH] if query.is_cuda \
         else [SDPBackend.MATH]

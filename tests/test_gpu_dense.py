@@ -1,0 +1,68 @@
+"""Dense attention of the warm-up branch (processor.dense_attention) on the sparse kernel: lengths at
+the edges of its key tiles, row blocks and items, both item sizes, the persistent grid, layouts,
+and the calls that stay with SDPA. The reference is float32 softmax attention per segment; bounds
+are those of the attention tests (P and the output are rounded to 16 bits)."""
+import pytest
+import torch
+
+from peco_amd import attention_cuda, processor
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _reference(q, k, v, valid):
+    out = torch.empty(q.shape, device=q.device)
+    for a, b in ((0, valid), (valid, q.shape[2])):
+        if a < b:
+            for h in range(q.shape[1]):  # head by head: small score matrices
+                s = q[:, h, a:b].float() @ k[:, h, a:b].float().transpose(1, 2).contiguous() * q.shape[3] ** -0.5
+                out[:, h, a:b] = torch.softmax(s, -1) @ v[:, h, a:b].float()
+    return out
+
+
+def _inputs(batch, heads, length, dim, dtype):
+    g = torch.Generator(device=DEV)
+    g.manual_seed(length + heads)
+    return [torch.randn(batch, heads, length, dim, generator=g, device=DEV).to(dtype) for _ in range(3)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("batch,heads,length,dim,valid", [
+    (1, 1, 1, 128, 1), (1, 2, 63, 64, 0), (1, 2, 64, 128, 64), (2, 3, 65, 128, 64), (1, 3, 129, 64, 1),
+    (1, 2, 257, 128, 128), (1, 2, 1000, 128, 937),
+    (1, 64, 2309, 64, 2100),    # 256-row items on 8-wavefront workgroups
+    (1, 64, 4300, 128, 4250),   # the same on the persistent grid
+    (10, 200, 70, 64, 40),      # 128-row items on the persistent grid
+])
+def test_dense_attention_matches_reference(dtype, batch, heads, length, dim, valid):
+    q, k, v = _inputs(batch, heads, length, dim, dtype)
+    assert attention_cuda.dense_supported(q, k, v, valid)
+    ref = _reference(q, k, v, valid)
+    for _ in range(2):  # the second call finds the workspace as the first left it
+        err = (processor.dense_attention(q, k, v, valid).float() - ref).abs()
+        assert err.max().item() <= 2e-2 and err.mean().item() <= 2e-3
+
+
+def test_dense_attention_keeps_layout_and_sdpa_calls():
+    q, k, v = (t.transpose(1, 2).contiguous().transpose(1, 2) for t in _inputs(1, 4, 200, 64, torch.bfloat16))
+    out = processor.dense_attention(q, k, v, 150)
+    assert out.stride() == torch.empty_like(q).stride()
+    assert (out.float() - _reference(q, k, v, 150)).abs().max().item() <= 2e-2
+    # Gradients, other head dimensions and float32 are SDPA's.
+    leaf = q.clone().requires_grad_(True)
+    processor.dense_attention(leaf, k, v, 150).float().sum().backward()
+    assert leaf.grad is not None and torch.isfinite(leaf.grad).all()
+    for dim, dtype in ((32, torch.bfloat16), (64, torch.float32)):
+        a, b, c = _inputs(1, 2, 90, dim, dtype)
+        assert not attention_cuda.dense_supported(a, b, c, 60)
+        assert (processor.dense_attention(a, b, c, 60).float() - _reference(a, b, c, 60)).abs().max().item() <= 2e-2
+
+
+def test_dense_attention_padding_segment_sees_no_video_value():
+    """A non-finite value row is seen by its own segment only, also where a key tile is partial."""
+    q, k, v = _inputs(1, 2, 300, 128, torch.bfloat16)
+    v[0, 0, 0] = float("inf")
+    out = processor.dense_attention(q, k, v, 250)
+    assert torch.isfinite(out[0, 0, 250:]).all() and torch.isfinite(out[0, 1]).all()
+    assert not torch.isfinite(out[0, 0, :250]).any()
