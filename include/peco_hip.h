@@ -71,6 +71,14 @@ size_t peco_cluster_sort_workspace_size(int batch, int tokens, int clusters);
 int peco_cluster_sort(const int32_t* labels, int batch, int tokens, int clusters, int32_t* indices, int32_t* ranks,
                       int32_t* counts, int32_t* offsets, void* workspace, size_t workspace_bytes, void* stream);
 
+/* Stable argsort of integer labels [batch, tokens] of any value (label_bytes 4: int32, 8: int64) per
+ * batch entry (the torch.argsort of peco/clustering.py:105 where the label range is unknown):
+ * indices[b,j] = original token at sorted position j. No host synchronization; workspace 8-byte
+ * aligned. */
+size_t peco_label_argsort_workspace_size(int batch, int tokens);
+int peco_label_argsort(const void* labels, int label_bytes, int batch, int tokens, int32_t* indices, void* workspace,
+                       size_t workspace_bytes, void* stream);
+
 /* Fused Lloyd fit (peco/clustering.py:17-89 with tol=0) of num_problems (1 or 2)
  * independent problems. The problems' batch entries run as four chains of launches, three of
  * them on library-owned streams of the current device, forked from `stream` and joined back to

@@ -113,6 +113,8 @@ SIGNATURES = {
     "peco_abi_version": (I, []),
     "peco_cluster_sort_workspace_size": (Z, [I, I, I]),
     "peco_cluster_sort": (I, [P, I, I, I, P, P, P, P, P, Z, P]),
+    "peco_label_argsort_workspace_size": (Z, [I, I]),
+    "peco_label_argsort": (I, [P, I, I, I, P, P, Z, P]),
     "peco_kmeans_workspace_size": (Z, [I, I, I, I]),
     "peco_kmeans_fit": (I, [I, PP, P, PP, PP, PP, PP, PP, PP, IP, IP, IP, I, I, I, P, Z, P]),
     "peco_kmeans_screen": (I, [P, I, P, P, P, P, I, I, I, I, P]),

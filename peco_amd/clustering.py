@@ -11,7 +11,7 @@ import math
 
 import torch
 
-from . import clustering_cuda
+from . import _native, clustering_cuda
 
 
 def _require_gpu(*tensors):
@@ -82,7 +82,11 @@ def _prepare_sequence_indices(tensor, labels, dim, sorted_indices):
         if labels is None or labels.numel() != batch * heads * tokens or labels.device != tensor.device:
             raise ValueError("labels must contain one cluster ID per token on the same device")
         # Stable sort keeps the original order inside each cluster.
-        sorted_indices = torch.argsort(labels.reshape(batch * heads, tokens), dim=-1, stable=True)
+        rows = labels.reshape(batch * heads, tokens)
+        if rows.is_cuda and rows.dtype in (torch.int32, torch.int64) and _native.plain_tensors(rows) and \
+                clustering_cuda.label_argsort_fits(*rows.shape):
+            return clustering_cuda.label_argsort(rows)
+        sorted_indices = torch.argsort(rows, dim=-1, stable=True)
     if sorted_indices.numel() != batch * heads * tokens or sorted_indices.device != tensor.device:
         raise ValueError("sorted_indices must contain one index per token on the same device")
     return sorted_indices.reshape(batch * heads, tokens).to(torch.int32).contiguous()

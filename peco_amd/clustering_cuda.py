@@ -115,6 +115,29 @@ def cluster_sort(labels, clusters):
     return indices, counts, offsets
 
 
+def label_argsort_fits(batch, tokens):
+    """Whether label_argsort is worth its workspace (16 KB and more per entry, most of it digit
+    histograms): always up to 256 MB, which many thousand short entries would pass."""
+    return _library().peco_label_argsort_workspace_size(batch, tokens) <= 1 << 28
+
+
+def label_argsort(labels):
+    """Stable argsort of int32 or int64 labels [B,N] of any value: int32 indices [B,N], equal to
+    torch.argsort(labels, dim=-1, stable=True) (peco/clustering.py:105). No host synchronization."""
+    library = _library()
+    labels = labels.contiguous()
+    batch, tokens = labels.shape
+    indices = torch.empty((batch, tokens), dtype=torch.int32, device=labels.device)
+    ws_bytes = library.peco_label_argsort_workspace_size(batch, tokens)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=labels.device)
+    with torch.cuda.device(labels.device):
+        status = library.peco_label_argsort(
+            _native.ptr(labels), labels.element_size(), batch, tokens, _native.ptr(indices), _native.ptr(ws), ws_bytes,
+            _retain_on_current_stream(labels.device, labels, indices, ws))
+    _raise_cluster_error(status)
+    return indices
+
+
 class KMeansProblem:
     """One k-means problem for :func:`kmeans_fit`: x [B,N,D] (rows may have a batch stride)."""
 
