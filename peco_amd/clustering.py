@@ -83,8 +83,7 @@ def _prepare_sequence_indices(tensor, labels, dim, sorted_indices):
             raise ValueError("labels must contain one cluster ID per token on the same device")
         # Stable sort keeps the original order inside each cluster.
         rows = labels.reshape(batch * heads, tokens)
-        if rows.is_cuda and rows.dtype in (torch.int32, torch.int64) and _native.plain_tensors(rows) and \
-                clustering_cuda.label_argsort_fits(*rows.shape):
+        if rows.is_cuda and rows.dtype in (torch.int32, torch.int64) and _native.plain_tensors(rows):
             return clustering_cuda.label_argsort(rows)
         sorted_indices = torch.argsort(rows, dim=-1, stable=True)
     if sorted_indices.numel() != batch * heads * tokens or sorted_indices.device != tensor.device:

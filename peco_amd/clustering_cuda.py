@@ -115,12 +115,6 @@ def cluster_sort(labels, clusters):
     return indices, counts, offsets
 
 
-def label_argsort_fits(batch, tokens):
-    """Whether label_argsort is worth its workspace (16 KB and more per entry, most of it digit
-    histograms): always up to 256 MB, which many thousand short entries would pass."""
-    return _library().peco_label_argsort_workspace_size(batch, tokens) <= 1 << 28
-
-
 def label_argsort(labels):
     """Stable argsort of int32 or int64 labels [B,N] of any value: int32 indices [B,N], equal to
     torch.argsort(labels, dim=-1, stable=True) (peco/clustering.py:105). No host synchronization."""

@@ -325,49 +325,68 @@ __global__ __launch_bounds__(256) void sort_fused_kernel(SortArgs args) {
     }
 }
 
-// Stable argsort of labels whose range the host does not know (gather_clustered_tokens by labels):
-// an LSD radix sort whose digit width is chosen on the device from each entry's smallest and
-// largest label, so cluster labels (up to 2048 of them) take one pass and any 32- or 64-bit
-// values the 3 or 6 passes that are always launched; the passes an entry does not need return at
-// once. No host synchronization.
-//   label_range: per entry {min, digit bits, passes};
-//   per pass: digit histogram per chunk of kRadixChunk tokens; per entry the exclusive prefixes of
-//   the chunks and the digits' starts; placement, where a chunk's four wavefronts count their own
-//   stretch again and rank it 64 tokens at a time (place_step, as the counting sort above).
-// Latency-bound (a few dependent loads per launch): 24 x 32640 labels in 512 clusters about 35 us
-// (range 6, histogram 8, scan 8, placement 13); torch's merge sort took 325 us with its 20 launches
-// and the index conversion.
+// Stable argsort of labels whose range the host does not know (gather_clustered_tokens by labels),
+// without a host synchronization. Two forms, both latency-bound:
+//   block form, one launch: a workgroup sorts an entry by an LSD radix sort of up to 8-bit digits
+//     whose number and width follow from the entry's smallest and largest label (found first).
+//     Entries of at most kBlockSortTokens tokens take it: more launches would cost more than they
+//     spread;
+//   chunk form, for longer entries: the label range per entry, then one pass (up to kRadixBins
+//     different labels) or two of: the digit histogram per chunk of kRadixChunk tokens, per entry
+//     the exclusive prefixes of the chunks and the digits' starts, and the placement, where a
+//     chunk's four wavefronts count their own stretch again and rank it 64 tokens at a time
+//     (place_step, as the counting sort above). The second pass's launches return at once for
+//     entries that need one, and entries of more than 2 * kRadixBits bits are left to the block form
+//     in a last launch.
+// 24 x 32640 labels in 300 clusters: 32 us; torch's merge sort took 320 us with its 20 launches and the
+// index conversion. The line between the forms, 24 entries: 12000 tokens 29 us by blocks and 31-34
+// by chunks, 16384 tokens 37 and 32.
 constexpr int kRadixChunk = 2048;
 constexpr int kRadixWaves = 4;
 constexpr int kRadixBits = 11;
 constexpr int kRadixBins = 1 << kRadixBits;
+constexpr int kBlockSortTokens = 12288;
+constexpr int kBlockWaves = 16;
+constexpr int kBlockBits = 8;
 
 struct LabelRange {
     int64_t base;
-    int32_t bits, passes;
+    int32_t width;  // bits of (largest - smallest), at least 1
+    int32_t pad;
 };
 
 struct RadixArgs {
     const void* labels;   // [batch, tokens]
     int32_t* indices;     // [batch, tokens]
     int32_t* tmp[2];      // [batch, tokens] orders between passes
-    int32_t* hist;        // [batch, chunks, kRadixBins]
+    int32_t* hist;        // [batch, chunks, kRadixBins] (chunk form)
     int32_t* starts;      // [batch, kRadixBins]
     LabelRange* range;    // [batch]
-    int batch, tokens, chunks, pass;
+    int batch, tokens, chunks;
+    int pass;             // chunk form: 0 or 1
 };
 
+// Digit width of a chunk-form pass for labels of `width` bits, or 0 when the pass does nothing.
+__device__ __forceinline__ int chunk_bits(int width, int pass) {
+    if (width > 2 * kRadixBits || (pass == 1 && width <= kRadixBits)) return 0;
+    return width <= kRadixBits ? width : (width + 1) / 2;
+}
+
+// Token at position t of the order the pass starts from.
+__device__ __forceinline__ int radix_source(const RadixArgs& a, int b, int t) {
+    return a.pass == 0 ? t : a.tmp[0][static_cast<int64_t>(b) * a.tokens + t];
+}
+
+// Smallest label and width of one entry, by a workgroup of kBlockWaves wavefronts.
 template <typename L>
-__global__ __launch_bounds__(1024) void label_range_kernel(RadixArgs a) {
-    __shared__ L red[2][16];
-    const int b = blockIdx.x;
-    const L* lab = static_cast<const L*>(a.labels) + static_cast<int64_t>(b) * a.tokens;
+__device__ __forceinline__ LabelRange label_range(const L* lab, int tokens, L (&red)[2][kBlockWaves]) {
+    constexpr int NT = kBlockWaves * kWave;
     constexpr int U = 8;
     L lo = lab[0], hi = lo;
-    for (int t0 = threadIdx.x; t0 < a.tokens; t0 += U * 1024) {
+    for (int t0 = threadIdx.x; t0 < tokens; t0 += U * NT) {
         L v[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) v[u] = lab[min(t0 + u * 1024, a.tokens - 1)];  // clamped: all in flight
+        for (int u = 0; u < U; ++u) v[u] = lab[min(t0 + u * NT, tokens - 1)];  // clamped: all in flight
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             lo = v[u] < lo ? v[u] : lo;
@@ -385,27 +404,26 @@ __global__ __launch_bounds__(1024) void label_range_kernel(RadixArgs a) {
         red[1][threadIdx.x / kWave] = hi;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < 16; ++w) {
-            lo = red[0][w] < lo ? red[0][w] : lo;
-            hi = red[1][w] > hi ? red[1][w] : hi;
-        }
-        const uint64_t span = static_cast<uint64_t>(static_cast<int64_t>(hi)) - static_cast<uint64_t>(static_cast<int64_t>(lo));
-        const int width = span ? 64 - __builtin_clzll(span) : 1;
-        const int passes = (width + kRadixBits - 1) / kRadixBits;
-        a.range[b] = LabelRange{static_cast<int64_t>(lo), (width + passes - 1) / passes, passes};
+    for (int w = 0; w < kBlockWaves; ++w) {
+        lo = red[0][w] < lo ? red[0][w] : lo;
+        hi = red[1][w] > hi ? red[1][w] : hi;
     }
+    const uint64_t span = static_cast<uint64_t>(static_cast<int64_t>(hi)) - static_cast<uint64_t>(static_cast<int64_t>(lo));
+    return LabelRange{static_cast<int64_t>(lo), span ? 64 - __builtin_clzll(span) : 1, 0};
+}
+
+// Bits [shift, shift + bits) of a label's distance from the smallest one.
+template <typename L> __device__ __forceinline__ int label_digit(L label, int64_t base, int shift, int bits) {
+    const uint64_t d = static_cast<uint64_t>(static_cast<int64_t>(label)) - static_cast<uint64_t>(base);
+    return static_cast<int>((d >> shift) & ((1u << bits) - 1u));
 }
 
 template <typename L>
-__device__ __forceinline__ int label_digit(L label, const LabelRange& r, int pass) {
-    const uint64_t d = static_cast<uint64_t>(static_cast<int64_t>(label)) - static_cast<uint64_t>(r.base);
-    return static_cast<int>((d >> (pass * r.bits)) & ((1u << r.bits) - 1u));
-}
-
-// Token at position t of the order the pass starts from.
-__device__ __forceinline__ int radix_source(const RadixArgs& a, int b, int t) {
-    return a.pass == 0 ? t : a.tmp[(a.pass - 1) & 1][static_cast<int64_t>(b) * a.tokens + t];
+__global__ __launch_bounds__(kBlockWaves* kWave) void label_range_kernel(RadixArgs a) {
+    __shared__ L red[2][kBlockWaves];
+    const LabelRange r = label_range(static_cast<const L*>(a.labels) + static_cast<int64_t>(blockIdx.x) * a.tokens,
+                                     a.tokens, red);
+    if (threadIdx.x == 0) a.range[blockIdx.x] = r;
 }
 
 template <typename L>
@@ -413,38 +431,39 @@ __global__ __launch_bounds__(kRadixWaves * kWave) void radix_hist_kernel(RadixAr
     __shared__ int hist[kRadixBins];
     const int b = blockIdx.x / a.chunks, chunk = blockIdx.x % a.chunks;
     const LabelRange r = a.range[b];
-    if (a.pass >= r.passes) return;
-    const int bins = 1 << r.bits;
+    const int bits = chunk_bits(r.width, a.pass);
+    if (bits == 0) return;
+    const int bins = 1 << bits;
     for (int k = threadIdx.x; k < bins; k += blockDim.x) hist[k] = 0;
     __syncthreads();
     const L* lab = static_cast<const L*>(a.labels) + static_cast<int64_t>(b) * a.tokens;
     constexpr int U = kRadixChunk / (kRadixWaves * kWave);
+    const int t0 = chunk * kRadixChunk + static_cast<int>(threadIdx.x);
     int src[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u)
-        src[u] = radix_source(a, b, min(chunk * kRadixChunk + u * kRadixWaves * kWave + static_cast<int>(threadIdx.x),
-                                        a.tokens - 1));
+    for (int u = 0; u < U; ++u) src[u] = radix_source(a, b, min(t0 + u * kRadixWaves * kWave, a.tokens - 1));
     L v[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) v[u] = lab[src[u]];
 #pragma unroll
     for (int u = 0; u < U; ++u)
-        if (chunk * kRadixChunk + u * kRadixWaves * kWave + static_cast<int>(threadIdx.x) < a.tokens)
-            atomicAdd(&hist[label_digit(v[u], r, a.pass)], 1);
+        if (t0 + u * kRadixWaves * kWave < a.tokens)
+            atomicAdd(&hist[label_digit(v[u], r.base, a.pass * bits, bits)], 1);
     __syncthreads();
     int32_t* out = a.hist + (static_cast<int64_t>(b) * a.chunks + chunk) * kRadixBins;
     for (int k = threadIdx.x; k < bins; k += blockDim.x) out[k] = hist[k];
 }
 
-// Per entry: each (chunk, digit) count becomes its exclusive prefix over the chunks, and starts
-// receives the digits' first positions.
+// Per entry: each (chunk, label) count becomes its exclusive prefix over the chunks, and starts
+// receives the labels' first positions.
 __global__ __launch_bounds__(1024) void radix_scan_kernel(RadixArgs a) {
     __shared__ int total[kRadixBins];
     __shared__ int wave_sum[16];
     const int b = blockIdx.x;
     const LabelRange r = a.range[b];
-    if (a.pass >= r.passes) return;
-    const int bins = 1 << r.bits;
+    const int bits = chunk_bits(r.width, a.pass);
+    if (bits == 0) return;
+    const int bins = 1 << bits;
     int32_t* hist = a.hist + static_cast<int64_t>(b) * a.chunks * kRadixBins;
     constexpr int U = 8;
     for (int k = threadIdx.x; k < kRadixBins; k += 1024) {
@@ -467,7 +486,7 @@ __global__ __launch_bounds__(1024) void radix_scan_kernel(RadixArgs a) {
         total[k] = run;
     }
     __syncthreads();
-    // Exclusive scan of the digit totals: two adjacent digits per thread.
+    // Exclusive scan of the label totals: two adjacent labels per thread.
     const int x = total[2 * threadIdx.x], y = total[2 * threadIdx.x + 1];
     const int incl = wave_inclusive_scan(x + y);
     const int wave = threadIdx.x / kWave;
@@ -485,8 +504,9 @@ __global__ __launch_bounds__(kRadixWaves * kWave) void radix_place_kernel(RadixA
     __shared__ int base[kRadixWaves][kRadixBins];
     const int b = blockIdx.x / a.chunks, chunk = blockIdx.x % a.chunks;
     const LabelRange r = a.range[b];
-    if (a.pass >= r.passes) return;
-    const int bins = 1 << r.bits;
+    const int bits = chunk_bits(r.width, a.pass);
+    if (bits == 0) return;
+    const int bins = 1 << bits;
     const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
     for (int i = threadIdx.x; i < kRadixWaves * bins; i += blockDim.x) base[i / bins][i % bins] = 0;
     const L* lab = static_cast<const L*>(a.labels) + static_cast<int64_t>(b) * a.tokens;
@@ -501,7 +521,7 @@ __global__ __launch_bounds__(kRadixWaves * kWave) void radix_place_kernel(RadixA
 #pragma unroll
         for (int u = 0; u < kSteps; ++u) v[u] = lab[src[u]];
 #pragma unroll
-        for (int u = 0; u < kSteps; ++u) digit[u] = label_digit(v[u], r, a.pass);
+        for (int u = 0; u < kSteps; ++u) digit[u] = label_digit(v[u], r.base, a.pass * bits, bits);
     }
     __syncthreads();
 #pragma unroll
@@ -520,11 +540,91 @@ __global__ __launch_bounds__(kRadixWaves * kWave) void radix_place_kernel(RadixA
         }
     }
     __syncthreads();
-    int32_t* out = (a.pass + 1 == r.passes ? a.indices : a.tmp[a.pass & 1]) + static_cast<int64_t>(b) * a.tokens;
+    const bool last = a.pass == 1 || r.width <= kRadixBits;
+    int32_t* out = (last ? a.indices : a.tmp[0]) + static_cast<int64_t>(b) * a.tokens;
 #pragma unroll
     for (int u = 0; u < kSteps; ++u) {
-        const int pos = place_step(digit[u], first + u * kWave + lane < a.tokens, bins, r.bits, base[wave]);
+        const int pos = place_step(digit[u], first + u * kWave + lane < a.tokens, bins, bits, base[wave]);
         if (pos >= 0) out[pos] = src[u];
+    }
+}
+
+// The block form. kRest: only the entries the chunk form left (their range is known).
+template <typename L, bool kRest>
+__global__ __launch_bounds__(kBlockWaves* kWave) void block_argsort_kernel(RadixArgs a) {
+    __shared__ L red[2][kBlockWaves];
+    __shared__ int hist[kBlockWaves][1 << kBlockBits];
+    __shared__ int wave_sum[kBlockWaves];
+    const int b = blockIdx.x;
+    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    const L* lab = static_cast<const L*>(a.labels) + static_cast<int64_t>(b) * a.tokens;
+    LabelRange r;
+    if constexpr (kRest) {
+        r = a.range[b];
+        if (r.width <= 2 * kRadixBits) return;
+    } else {
+        r = label_range(lab, a.tokens, red);
+    }
+    const int passes = (r.width + kBlockBits - 1) / kBlockBits;
+    const int bits = (r.width + passes - 1) / passes;
+    const int bins = 1 << bits;
+    // Wavefront w holds positions [w * per, (w + 1) * per) of the order.
+    constexpr int U = 4;
+    const int per = static_cast<int>(ceil_div(a.tokens, kBlockWaves * kWave * U)) * kWave * U;
+    const int begin = min(a.tokens, wave * per), end = min(a.tokens, begin + per);
+    const int64_t row = static_cast<int64_t>(b) * a.tokens;
+    for (int pass = 0; pass < passes; ++pass) {
+        const int32_t* from = pass == 0 ? nullptr : a.tmp[(pass - 1) & 1] + row;
+        int32_t* to = (pass + 1 == passes ? a.indices : a.tmp[pass & 1]) + row;
+        for (int i = threadIdx.x; i < kBlockWaves * bins; i += blockDim.x) hist[i / bins][i % bins] = 0;
+        __syncthreads();
+        auto load = [&](int t0, int (&src)[U], int (&digit)[U]) {
+            L v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int t = min(t0 + u * kWave + lane, a.tokens - 1);
+                src[u] = from ? from[t] : t;
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) v[u] = lab[src[u]];
+#pragma unroll
+            for (int u = 0; u < U; ++u) digit[u] = label_digit(v[u], r.base, pass * bits, bits);
+        };
+        for (int t0 = begin; t0 < end; t0 += U * kWave) {
+            int src[U], digit[U];
+            load(t0, src, digit);
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (t0 + u * kWave + lane < end) atomicAdd(&hist[wave][digit[u]], 1);
+        }
+        __syncthreads();
+        // Starts: wavefronts' counts of a digit in turn, digits in order (one thread per digit).
+        int total = 0;
+        if (static_cast<int>(threadIdx.x) < bins)
+            for (int w = 0; w < kBlockWaves; ++w) total += hist[w][threadIdx.x];
+        const int incl = wave_inclusive_scan(total);
+        if (lane == kWave - 1) wave_sum[wave] = incl;
+        __syncthreads();
+        if (static_cast<int>(threadIdx.x) < bins) {
+            int run = incl - total;
+            for (int w = 0; w < wave; ++w) run += wave_sum[w];
+            for (int w = 0; w < kBlockWaves; ++w) {
+                const int n = hist[w][threadIdx.x];
+                hist[w][threadIdx.x] = run;
+                run += n;
+            }
+        }
+        __syncthreads();
+        for (int t0 = begin; t0 < end; t0 += U * kWave) {
+            int src[U], digit[U];
+            load(t0, src, digit);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int pos = place_step(digit[u], t0 + u * kWave + lane < end, bins, bits, hist[wave]);
+                if (pos >= 0) to[pos] = src[u];
+            }
+        }
+        __syncthreads();  // the order is complete (and the counts are free) before the next pass
     }
 }
 
@@ -619,8 +719,9 @@ PECO_API int peco_cluster_sort(const int32_t* labels, int batch, int tokens, int
 
 // int32 elements of peco_label_argsort's workspace.
 static size_t radix_workspace_ints(int batch, int tokens) {
-    const size_t b = static_cast<size_t>(batch), chunks = static_cast<size_t>(ceil_div(tokens, kRadixChunk));
-    return b * 4 + b * (chunks + 1) * kRadixBins + 2 * b * tokens;
+    const size_t b = static_cast<size_t>(batch);
+    const size_t chunks = tokens > kBlockSortTokens ? static_cast<size_t>(ceil_div(tokens, kRadixChunk)) : 0;
+    return (chunks ? b * 4 + b * (chunks + 1) * kRadixBins : 0) + 2 * b * tokens;
 }
 
 PECO_API size_t peco_label_argsort_workspace_size(int batch, int tokens) {
@@ -638,24 +739,32 @@ PECO_API int peco_label_argsort(const void* labels, int label_bytes, int batch, 
     a.indices = indices;
     a.batch = batch;
     a.tokens = tokens;
-    a.chunks = static_cast<int>(ceil_div(tokens, kRadixChunk));
-    if (static_cast<int64_t>(batch) * a.chunks > 0x7fffffff) return kUnsupportedShape;
     int32_t* ws = static_cast<int32_t*>(workspace);
-    a.range = reinterpret_cast<LabelRange*>(ws);
-    a.starts = ws + static_cast<size_t>(batch) * 4;
-    a.hist = a.starts + static_cast<size_t>(batch) * kRadixBins;
-    a.tmp[0] = a.hist + static_cast<size_t>(batch) * a.chunks * kRadixBins;
-    a.tmp[1] = a.tmp[0] + static_cast<size_t>(batch) * tokens;
+    if (tokens > kBlockSortTokens) {
+        a.chunks = static_cast<int>(ceil_div(tokens, kRadixChunk));
+        if (static_cast<int64_t>(batch) * a.chunks > 0x7fffffff) return kUnsupportedShape;
+        a.range = reinterpret_cast<LabelRange*>(ws);
+        a.starts = ws + static_cast<size_t>(batch) * 4;
+        a.hist = a.starts + static_cast<size_t>(batch) * kRadixBins;
+        ws = a.hist + static_cast<size_t>(batch) * a.chunks * kRadixBins;
+    }
+    a.tmp[0] = ws;
+    a.tmp[1] = ws + static_cast<size_t>(batch) * tokens;
     const auto s = static_cast<hipStream_t>(stream);
     auto launch = [&](auto tag) {
         using L = decltype(tag);
-        hipLaunchKernelGGL(label_range_kernel<L>, dim3(batch), dim3(1024), 0, s, a);
-        const int passes = (8 * static_cast<int>(sizeof(L)) + kRadixBits - 1) / kRadixBits;
-        for (a.pass = 0; a.pass < passes; ++a.pass) {
+        const dim3 block(kBlockWaves * kWave);
+        if (tokens <= kBlockSortTokens) {
+            hipLaunchKernelGGL((block_argsort_kernel<L, false>), dim3(batch), block, 0, s, a);
+            return;
+        }
+        hipLaunchKernelGGL(label_range_kernel<L>, dim3(batch), block, 0, s, a);
+        for (a.pass = 0; a.pass < 2; ++a.pass) {
             hipLaunchKernelGGL(radix_hist_kernel<L>, dim3(batch * a.chunks), dim3(kRadixWaves * kWave), 0, s, a);
             hipLaunchKernelGGL(radix_scan_kernel, dim3(batch), dim3(1024), 0, s, a);
             hipLaunchKernelGGL(radix_place_kernel<L>, dim3(batch * a.chunks), dim3(kRadixWaves * kWave), 0, s, a);
         }
+        hipLaunchKernelGGL((block_argsort_kernel<L, true>), dim3(batch), block, 0, s, a);
     };
     if (label_bytes == 4) launch(int32_t{});
     else launch(int64_t{});
