@@ -55,6 +55,12 @@ int peco_sparse_attention(const void* q, const void* k, const void* v, const uin
                           const int* q_sizes, const int* k_sizes, void* output, int* workspace, int bh, int sq,
                           int sk, int d, int cq, int ck, int dtype, void* stream);
 
+/* Cluster size checks of the Python entry (peco/attention_cuda.py:101-110) in one launch: ok [4],
+ * set to 1 by the caller, is cleared where some head has a negative q size, a negative k size, q
+ * sizes not summing to sq, k sizes not summing to sk. */
+int peco_check_cluster_sizes(const int* q_sizes, const int* k_sizes, int bh, int cq, int ck, int sq, int sk,
+                             uint8_t* ok, void* stream);
+
 /* Replaces peco_attention_error_string, peco/kernels/sparse_attention.cu:232. */
 const char* peco_attention_error_string(int code);
 

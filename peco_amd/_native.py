@@ -133,6 +133,7 @@ SIGNATURES = {
     "peco_select_work_size": (Z, [I] * 5),
     "peco_select_work": (I, [P] * 4 + [I] * 4 + [ctypes.c_float] + [I] * 6 + [P] * 4 + [Z, P]),
     "peco_sparse_attention_work": (I, [P] * 5 + [I, P, P, I, I, P, Z] + [I] * 7 + [P]),
+    "peco_check_cluster_sizes": (I, [P, P] + [I] * 5 + [P, P]),
     "peco_dense_attention_workspace_size": (Z, [I, I]),
     "peco_dense_attention": (I, [P] * 4 + [I, P, Z] + [I] * 4 + [P]),
     "peco_place_heads": (I, [P] + [ctypes.c_int64] * 3 + [P] * 3 + [I] * 7 + [P]),

@@ -60,6 +60,19 @@ def _validate(q, k, v, dynamic_map, q_sizes, k_sizes):
     return batch, heads, sq, dim, sk, cq, ck, stride
 
 
+def _assert_sizes(q_sizes, k_sizes, bh, cq, ck, sq, sk):
+    """Asynchronous checks of the cluster sizes, on the stream (no copy to the host)."""
+    ok = torch.ones(4, dtype=torch.bool, device=q_sizes.device)
+    error = _native.library().peco_check_cluster_sizes(
+        _native.ptr(q_sizes), _native.ptr(k_sizes), bh, cq, ck, sq, sk, _native.ptr(ok),
+        _native.current_stream(q_sizes.device, q_sizes, k_sizes, ok))
+    _native.check(error, "PECO HIP cluster size check")
+    messages = ("q_sizes must be nonnegative", "k_sizes must be nonnegative",
+                "q_sizes must sum to the Q sequence length", "k_sizes must sum to the K sequence length")
+    for flag, message in zip(ok.unbind(), messages):
+        torch._assert_async(flag, message)
+
+
 def _check_index(index, name, batch, heads, rows):
     if not isinstance(index, torch.Tensor) or index.dtype != torch.int32 or not index.is_contiguous():
         raise ValueError(f"{name} must be a contiguous int32 tensor")
@@ -73,10 +86,7 @@ def _launch(q, k, v, dynamic_map, q_sizes, k_sizes, validate_sizes, out_index, k
         if not _device_is_gfx950(q.device):
             raise RuntimeError("This HIP build requires an MI355X-class gfx950 GPU")
         if validate_sizes:
-            torch._assert_async((q_sizes >= 0).all(), "q_sizes must be nonnegative")
-            torch._assert_async((k_sizes >= 0).all(), "k_sizes must be nonnegative")
-            torch._assert_async((q_sizes.sum(-1) == sq).all(), "q_sizes must sum to the Q sequence length")
-            torch._assert_async((k_sizes.sum(-1) == sk).all(), "k_sizes must sum to the K sequence length")
+            _assert_sizes(q_sizes, k_sizes, batch * heads, cq, ck, sq, sk)
         output = torch.empty_like(q)
         if sq == 0:
             return output

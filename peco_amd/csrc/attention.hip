@@ -4,7 +4,7 @@
 //   out_i = sum_{j : map[cq(i), ck(j)]} softmax_j(q_i.k_j / sqrt(D)) v_j, and 0 when row i
 //   keeps no key. Query and key rows are grouped by cluster in the order of q_sizes/k_sizes.
 //
-// Work list (one 256-thread workgroup per (batch*head)):
+// Work list (one 1024-thread workgroup per (batch*head)):
 //   cluster offsets are min(S, prefix of max(0, size)) (the reference's clamped running sum),
 //   each query cluster is cut into items of <= 128 rows (256 from 65536 query rows on), and the
 //   items of one head are ordered by descending cost rows * kept_keys. The attention grid is
@@ -57,21 +57,26 @@ __host__ __device__ inline WorkLayout work_layout(int32_t* ws, int bh, int sq, i
     return w;
 }
 
+// The builder runs one workgroup per head, few of them and latency-bound, so it takes as many
+// wavefronts as a workgroup can have: 12 heads of 90 x 331 clusters 16 us (24 us with four
+// wavefronts of 24 map rows each).
+constexpr int kBuildWaves = 16;
 // Map rows read per wavefront per pass, and bytes of a row per lane per pass (320 keys): one
-// pass covers a head of up to 96 query clusters and 320 key clusters.
-constexpr int kMapRows = 24;
+// pass covers a head of up to 128 query clusters and 320 key clusters.
+constexpr int kMapRows = 8;
 constexpr int kMapU = 5;
 
 // kGivenKept: kept_in [bh, cq] holds each query cluster's kept key rows (from the selection
 // launch), so the map is not read; the counts only order the items.
 template <bool kGivenKept>
-__global__ __launch_bounds__(256) void build_work_kernel(const uint8_t* __restrict__ selected,
+__global__ __launch_bounds__(kBuildWaves * kWave) void build_work_kernel(const uint8_t* __restrict__ selected,
                                                          const int* __restrict__ q_sizes,
                                                          const int* __restrict__ k_sizes,
                                                          const int32_t* __restrict__ kept_in, int32_t* ws, int bhn,
                                                          int sq, int sk, int cq, int ck, int tile) {
     extern __shared__ int lds[];
-    __shared__ int tmp[4];
+    constexpr int NT = kBuildWaves * kWave;
+    __shared__ int tmp[kBuildWaves];
     const int bh = blockIdx.x;
     const int wave = threadIdx.x / kWave, lane = lane_id();
     WorkLayout W = work_layout(ws, bhn, sq, cq, ck);
@@ -81,10 +86,10 @@ __global__ __launch_bounds__(256) void build_work_kernel(const uint8_t* __restri
     uint64_t* keys = reinterpret_cast<uint64_t*>(lds + ((ck + 2 * cq + 1 + 1) & ~1));  // [pow2 >= cap] sort keys
     int32_t* kpre = W.kprefix + static_cast<int64_t>(bh) * (ck + 1);
     const uint8_t* map = selected + static_cast<int64_t>(bh) * cq * ck;
-    // The map rows of wavefront w are w, w+4, ...; a pass covers kMapRows of them and kMapU*64
+    // The map rows of wavefront w are w, w + kBuildWaves, ...; a pass covers kMapRows of them and kMapU*64
     // keys, every byte load of the pass in flight at once. The first pass is issued before the
     // size scans so its latency overlaps them.
-    const int my_rows = cq > wave ? static_cast<int>(ceil_div(cq - wave, 4)) : 0;
+    const int my_rows = cq > wave ? static_cast<int>(ceil_div(cq - wave, kBuildWaves)) : 0;
     const int chunks = static_cast<int>(ceil_div(ck, kMapU * kWave));
     const int passes = kGivenKept ? 0 : static_cast<int>(ceil_div(my_rows, kMapRows)) * chunks;
     // Raw bytes, kept unmasked so that the loads stay in flight until the pass uses them: a
@@ -96,7 +101,7 @@ __global__ __launch_bounds__(256) void build_work_kernel(const uint8_t* __restri
         const int k0 = (pass % chunks) * kMapU * kWave;
 #pragma unroll
         for (int r = 0; r < kMapRows; ++r) {
-            const int c = min(wave + 4 * max(0, min(r0 + r, my_rows - 1)), cq - 1);
+            const int c = min(wave + kBuildWaves * max(0, min(r0 + r, my_rows - 1)), cq - 1);
             const uint8_t* row = map + static_cast<int64_t>(c) * ck;
 #pragma unroll
             for (int u = 0; u < kMapU; ++u) m[r][u] = row[min(k0 + u * kWave + lane, ck - 1)];
@@ -106,8 +111,8 @@ __global__ __launch_bounds__(256) void build_work_kernel(const uint8_t* __restri
     // are issued before the first map pass: loads complete in order, so the size scans below
     // then wait only for these.
     constexpr int kSizes = 4;
-    const int kper = static_cast<int>(ceil_div(ck, 256));
-    const int qper = static_cast<int>(ceil_div(cq, 256));
+    const int kper = static_cast<int>(ceil_div(ck, NT));
+    const int qper = static_cast<int>(ceil_div(cq, NT));
     int kv[kSizes], qv[kSizes];
     if (kper <= kSizes && qper <= kSizes) {
 #pragma unroll
@@ -140,7 +145,7 @@ __global__ __launch_bounds__(256) void build_work_kernel(const uint8_t* __restri
             }
         }
         int total;
-        int run = block_scan<4>(local, tmp, &total);
+        int run = block_scan<kBuildWaves>(local, tmp, &total);
         for (int c = c0; c < c1; ++c) {
             const int a = min(sk, run);
             run += ksz[c];
@@ -171,7 +176,7 @@ __global__ __launch_bounds__(256) void build_work_kernel(const uint8_t* __restri
             }
         }
         int total;
-        int run = block_scan<4>(local, tmp, &total);
+        int run = block_scan<kBuildWaves>(local, tmp, &total);
         for (int c = c0; c < c1; ++c) {
             const int v = qoff[c];
             qoff[c] = min(sq, run);
@@ -202,13 +207,12 @@ __global__ __launch_bounds__(256) void build_work_kernel(const uint8_t* __restri
         if (pass + 1 < passes) issue(pass + 1);
 #pragma unroll
         for (int r = 0; r < kMapRows; ++r) {
-#pragma unroll
-            for (int o = 1; o < kWave; o <<= 1) sum[r] += __shfl_xor(sum[r], o, kWave);
-            if (lane == 0 && r0 + r < my_rows) kept[wave + 4 * (r0 + r)] += sum[r];
+            sum[r] = wave_incl_scan(sum[r]);  // the last lane holds the row's sum
+            if (lane == kWave - 1 && r0 + r < my_rows) kept[wave + kBuildWaves * (r0 + r)] += sum[r];
         }
     }
     __syncthreads();
-    order_head_items<4>(qoff, kept, cq, tile, W.items + static_cast<int64_t>(bh) * W.cap * 3, W.counts + bh, keys,
+    order_head_items<kBuildWaves>(qoff, kept, cq, tile, W.items + static_cast<int64_t>(bh) * W.cap * 3, W.counts + bh, keys,
                         tmp);
 }
 
@@ -1414,10 +1418,10 @@ int launch_sparse_attention(const void* q, const void* k, const void* v, const u
     if (lds_build > 60 * 1024 || lds_attn > 24 * 1024) return kUnsupportedShape;
     const hipStream_t s = static_cast<hipStream_t>(stream);
     if (kept_keys)
-        hipLaunchKernelGGL(build_work_kernel<true>, dim3(bh), dim3(256), lds_build, s, selected, q_sizes, k_sizes,
+        hipLaunchKernelGGL(build_work_kernel<true>, dim3(bh), dim3(kBuildWaves * kWave), lds_build, s, selected, q_sizes, k_sizes,
                            kept_keys, workspace, bh, sq, sk, cq, ck, attention_item_rows(sq));
     else
-        hipLaunchKernelGGL(build_work_kernel<false>, dim3(bh), dim3(256), lds_build, s, selected, q_sizes, k_sizes,
+        hipLaunchKernelGGL(build_work_kernel<false>, dim3(bh), dim3(kBuildWaves * kWave), lds_build, s, selected, q_sizes, k_sizes,
                            nullptr, workspace, bh, sq, sk, cq, ck, attention_item_rows(sq));
     const WorkLayout W = work_layout(workspace, bh, sq, cq, ck);
     return launch_attention_kernel(q, k, v, selected, W.kprefix, nullptr, W.counts, W.items, W.cap, output, out_index,
@@ -1579,7 +1583,7 @@ PECO_API int peco_base_offset_attention(const void* q, const int32_t* out_index,
     if (lds_build > 60 * 1024 || lds_list > 24 * 1024) return kUnsupportedShape;
     const hipStream_t s = static_cast<hipStream_t>(stream);
     // The integer-score kernel runs 4-wavefront workgroups: items of kQTile rows.
-    hipLaunchKernelGGL(build_work_kernel<false>, dim3(bh), dim3(256), lds_build, s, selected, q_sizes, k_sizes, nullptr,
+    hipLaunchKernelGGL(build_work_kernel<false>, dim3(bh), dim3(kBuildWaves * kWave), lds_build, s, selected, q_sizes, k_sizes, nullptr,
                        workspace, bh, sq, sk, cq, ck, kQTile);
     const WorkLayout W = work_layout(workspace, bh, sq, cq, ck);
     BoAttnArgs a;
@@ -1623,6 +1627,51 @@ PECO_API int peco_base_offset_attention(const void* q, const int32_t* out_index,
         else PECO_BO(kF16, 64);
     }
 #undef PECO_BO
+    return hipGetLastError();
+}
+
+// Validity of the cluster sizes (peco/attention_cuda.py:101-110), one wavefront per (head, side): ok
+// [4] = q_sizes nonnegative, k_sizes nonnegative, q_sizes summing to sq, k_sizes to sk; set to 1
+// by the caller, cleared here where a head violates it (every writer writes 0). Stands for fourteen
+// small torch launches, 45 us of a 190 us call at 12 heads x 9361 rows.
+namespace peco {
+namespace {
+
+__global__ __launch_bounds__(256) void check_sizes_kernel(const int* __restrict__ q_sizes, const int* __restrict__ k_sizes,
+                                                          int bh, int cq, int ck, int sq, int sk, uint8_t* ok) {
+    const int lane = lane_id();
+    const int64_t w = static_cast<int64_t>(blockIdx.x) * 4 + threadIdx.x / kWave;
+    if (w >= 2 * static_cast<int64_t>(bh)) return;
+    const int side = w >= bh;
+    const int n = side ? ck : cq;
+    const int* sizes = (side ? k_sizes : q_sizes) + (w - (side ? bh : 0)) * n;
+    int64_t sum = 0;
+    bool negative = false;
+    for (int c0 = 0; c0 < n; c0 += 4 * kWave) {
+        int v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = sizes[min(c0 + u * kWave + lane, n - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (c0 + u * kWave + lane < n) {
+                sum += v[u];
+                negative = negative || v[u] < 0;
+            }
+    }
+#pragma unroll
+    for (int m = 1; m < kWave; m <<= 1) sum += __shfl_xor(static_cast<long long>(sum), m, kWave);
+    if (__any(negative) && lane == 0) ok[side] = 0;
+    if (sum != (side ? sk : sq) && lane == 0) ok[2 + side] = 0;
+}
+
+}  // namespace
+}  // namespace peco
+
+PECO_API int peco_check_cluster_sizes(const int* q_sizes, const int* k_sizes, int bh, int cq, int ck, int sq, int sk,
+                                      uint8_t* ok, void* stream) {
+    if (!q_sizes || !k_sizes || !ok || bh < 1 || cq < 1 || ck < 1) return kInvalidValue;
+    hipLaunchKernelGGL(check_sizes_kernel, dim3(static_cast<unsigned>(ceil_div(2 * static_cast<int64_t>(bh), 4))),
+                       dim3(256), 0, static_cast<hipStream_t>(stream), q_sizes, k_sizes, bh, cq, ck, sq, sk, ok);
     return hipGetLastError();
 }
 
