@@ -100,6 +100,18 @@ int peco_kmeans_fit(int num_problems, const void* const* x, const int64_t* x_bat
                     const int* batch, const int* tokens, const int* clusters, int dims, int dtype, int iterations,
                     void* workspace, size_t workspace_bytes, void* stream);
 
+/* Iterations [first, first + iterations) of a one-problem fit that stops once no centre moves further
+ * than tol (peco/clustering.py:61-86). Means of iteration i go to centers_a (i even) or centers_b
+ * (i odd); flags int32 [iterations + 1, 1 + batch], zeroed but for row 0: all 1 when first is 0,
+ * else the last row of the call before. Row t + 1 receives {1 if a centre moved past tol, per
+ * entry 1 if a centre changed} of iteration first + t; after a row whose first value stays 0 the
+ * later iterations change nothing (labels, counts, permutation and centres are that iteration's).
+ * The workspace (peco_kmeans_workspace_size) carries the fit between calls. */
+int peco_kmeans_iterate(const void* x, int64_t x_batch_stride, const float* centers_in, float* centers_a,
+                        float* centers_b, int32_t* labels, int32_t* counts, int32_t* sorted_indices, int32_t* offsets,
+                        int batch, int tokens, int clusters, int dims, int dtype, int first, int iterations, float tol,
+                        int32_t* flags, void* workspace, size_t workspace_bytes, void* stream);
+
 /* peco_kmeans_fit that also packs (fuses peco/processor.py:141-149 into the fit): for
  * problem i with hat[i] non-null, hat[i] [batch, length, dims] receives x's rows
  * Base-Offset fake-quantized with bits[i] (4 or 8) against the final centres, in the final

@@ -117,6 +117,7 @@ SIGNATURES = {
     "peco_label_argsort": (I, [P, I, I, I, P, P, Z, P]),
     "peco_kmeans_workspace_size": (Z, [I, I, I, I]),
     "peco_kmeans_fit": (I, [I, PP, P, PP, PP, PP, PP, PP, PP, IP, IP, IP, I, I, I, P, Z, P]),
+    "peco_kmeans_iterate": (I, [P, ctypes.c_int64] + [P] * 7 + [I] * 7 + [ctypes.c_float, P, P, Z, P]),
     "peco_kmeans_screen": (I, [P, I, P, P, P, P, I, I, I, I, P]),
     "peco_kmeans_screen_bound": (None, [I, P, P]),
     "peco_base_offset_encode": (I, [P, I, P, P, I, I, I, I, I, P, P, P, P]),

@@ -27,7 +27,7 @@ def fit_token_clusters(x, n_clusters, max_iters=100, tol=1e-4, init_centroids=No
     across denoising steps. Returns labels [BH,N] int32, centers [BH,K,D] fp32, counts
     [BH,K] int32 and the iteration count (peco/clustering.py:17-89). ``tol=0`` runs the
     fixed iteration count with no host synchronization; ``tol>0`` stops once the largest
-    centre displacement is <= tol (one host sync per iteration). ``chunk_size`` is
+    centre displacement is <= tol (a host sync every few iterations). ``chunk_size`` is
     validated for compatibility; the MFMA assignment needs no token chunking.
     """
     if x.ndim != 3 or not x.is_floating_point():
@@ -59,14 +59,7 @@ def fit_token_clusters(x, n_clusters, max_iters=100, tol=1e-4, init_centroids=No
         labels, centers, counts, _, _ = clustering_cuda.kmeans_fit(
             [clustering_cuda.KMeansProblem(x, centers)], max_iters)[0]
         return labels, centers, counts, max_iters
-    iteration = 0
-    for iteration in range(1, max_iters + 1):
-        labels, means, counts, _, _ = clustering_cuda.kmeans_fit([clustering_cuda.KMeansProblem(x, centers)], 1)[0]
-        shift = torch.linalg.vector_norm(means - centers, dim=-1).max().item()
-        centers = means
-        if shift <= tol:
-            break
-    return labels, centers, counts, iteration
+    return clustering_cuda.kmeans_fit_until(clustering_cuda.KMeansProblem(x, centers), max_iters, tol)
 
 
 def _prepare_sequence_indices(tensor, labels, dim, sorted_indices):

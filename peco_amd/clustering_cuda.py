@@ -255,6 +255,54 @@ def kmeans_fit(problems, iterations, pack=None, pack_order="cluster"):
     return outs, packed
 
 
+# Iterations of a converging fit launched between two looks at its flags: a look costs a host
+# synchronization (about 20 us with the launches behind it, half an iteration of the 480p features),
+# launches past the stop return at once.
+_TOL_STEP = 8
+
+
+def _float32_floor(value):
+    """Largest float32 not above value >= 0, so that comparing an fp32 number with it decides as
+    comparing with value itself."""
+    bits = ctypes.c_uint32.from_buffer_copy(ctypes.c_float(value)).value
+    if ctypes.c_float(value).value > value:
+        bits -= 1
+    return ctypes.c_float.from_buffer_copy(ctypes.c_uint32(bits)).value
+
+
+def kmeans_fit_until(problem, max_iters, tol):
+    """Lloyd iterations of one problem until the largest centre displacement is <= tol
+    (peco/clustering.py:61-86), at most max_iters. Returns (labels, centers, counts, iterations) as
+    one kmeans_fit call per iteration with a check in between gives them; the displacement is an fp32
+    norm."""
+    library = _library()
+    p, dims, dev = problem, problem.dims, problem.x.device
+    labels, indices = (torch.empty((p.batch, p.tokens), dtype=torch.int32, device=dev) for _ in range(2))
+    centers = [torch.empty((p.batch, p.clusters, dims), dtype=torch.float32, device=dev) for _ in range(2)]
+    counts = torch.empty((p.batch, p.clusters), dtype=torch.int32, device=dev)
+    offsets = torch.empty((p.batch, p.clusters + 1), dtype=torch.int32, device=dev)
+    ws_bytes = library.peco_kmeans_workspace_size(p.batch, p.tokens, p.clusters, dims)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+    done, last = 0, None
+    while done < max_iters:
+        step = min(_TOL_STEP, max_iters - done)
+        flags = torch.zeros((step + 1, 1 + p.batch), dtype=torch.int32, device=dev)
+        flags[0].fill_(1) if last is None else flags[0].copy_(last)
+        with torch.cuda.device(dev):
+            status = library.peco_kmeans_iterate(
+                _native.ptr(p.x), p.x.stride(0), _native.ptr(p.init), _native.ptr(centers[0]), _native.ptr(centers[1]),
+                _native.ptr(labels), _native.ptr(counts), _native.ptr(indices), _native.ptr(offsets), p.batch, p.tokens,
+                p.clusters, dims, _DTYPES[p.x.dtype], done, step, _float32_floor(tol), _native.ptr(flags), _native.ptr(ws),
+                ws_bytes, _retain_on_current_stream(dev, p.x, p.init))
+        _raise_cluster_error(status)
+        last = flags[step]
+        moved = flags[1:, 0].tolist()  # waits for these iterations
+        done += moved.index(0) + 1 if 0 in moved else step
+        if 0 in moved:
+            break
+    return labels, centers[(done - 1) % 2], counts, done
+
+
 def select_connections(query_centroids, key_centroids, q_counts, k_counts, p, minimum, text=None, *,
                        with_kept=False):
     """Cluster-pair map of select_cluster_connections in one launch.

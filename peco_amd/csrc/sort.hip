@@ -72,6 +72,7 @@ __global__ __launch_bounds__(256) void sort_scan_groups_kernel(SortArgs args) {
     const int local = blockIdx.x - P.scan_group_begin;
     const int b = local / P.scan_groups;
     const int g = local % P.scan_groups;
+    if (sort_skips(args, b)) return;
     const int K = P.clusters;
     const int t0 = g * kScanTiles;
     const int nt = min(kScanTiles, P.tiles - t0);
@@ -103,6 +104,7 @@ __global__ __launch_bounds__(256) void sort_scan_kernel(SortArgs args) {
     const int pi = find_problem_by_batch(args, blockIdx.x);
     const SortProblem& P = args.p[pi];
     const int b = blockIdx.x - P.batch_begin;
+    if (sort_skips(args, b)) return;
     const int K = P.clusters;
     const int groups = P.scan_groups;
     int32_t* gt = scan_group_area(P) + static_cast<int64_t>(b) * groups * K;
@@ -169,6 +171,7 @@ __global__ __launch_bounds__(64) void sort_place_kernel(SortArgs args) {
     const int local = blockIdx.x - P.block_begin;
     const int b = local / P.tiles;
     const int tile = local % P.tiles;
+    if (sort_skips(args, b)) return;
     const int K = P.clusters;
     const int lane = threadIdx.x;
     const int32_t* th = P.tile_hist + (static_cast<int64_t>(b) * P.tiles + tile) * K;
@@ -241,6 +244,7 @@ __global__ __launch_bounds__(256) void sort_fused_kernel(SortArgs args) {
     const int local = blockIdx.x - P.group_begin;
     const int b = local / groups;
     const int g = local % groups;
+    if (sort_skips(args, b)) return;
     const int K = P.clusters;
     const int tiles = P.tiles;
     const int wave = threadIdx.x / kWave;

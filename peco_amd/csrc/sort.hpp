@@ -35,9 +35,17 @@ struct SortArgs {
     int total_batches;  // sum of batch
     int zero_hist;      // sort_place clears each consumed tile histogram (for accumulating producers)
     int fused;          // one sort_fused launch instead of scan + place (sort_fusable problems only)
+    // Nullable (one problem only): {0 when nothing is left to do, entry b's flag}; entries whose flag
+    // is 0 are left as they are when skip_fixed is set (a k-means fit's settled entries).
+    const int32_t* settled;
+    int skip_fixed;
     int total_groups;   // sum of batch * ceil(tiles / kFusedTiles)
     int total_scan_groups;  // sum of batch * scan_groups
 };
+
+__device__ __forceinline__ bool sort_skips(const SortArgs& a, int b) {
+    return a.settled && (a.settled[0] == 0 || (a.skip_fixed && a.settled[1 + b] == 0));
+}
 
 // Fused sort: a workgroup ranks kFusedTiles consecutive tiles (one per wavefront) and derives
 // the cluster offsets of its batch entry from the tile histograms itself. Each workgroup reads
