@@ -86,7 +86,7 @@ int peco_label_argsort(const void* labels, int label_bytes, int batch, int token
                        size_t workspace_bytes, void* stream);
 
 /* Fused Lloyd fit (peco/clustering.py:17-89 with tol=0) of num_problems (1 or 2)
- * independent problems. The problems' batch entries run as four chains of launches, three of
+ * independent problems. A large fit's batch entries run as four chains of launches, three of
  * them on library-owned streams of the current device, forked from `stream` and joined back to
  * it with events, so the call is ordered on `stream` like a single chain. Problem i: x[i] rows [batch, tokens, dims]
  * in `dtype` with batch stride x_batch_stride[i] elements (NULL or 0 = tokens*dims),

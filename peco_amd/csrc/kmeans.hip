@@ -24,8 +24,8 @@
 // Per iteration: assign (+ per-tile label histogram via global atomics) -> sort scan ->
 // sort place (stable counting sort, also yields the final permutation for stage 3) ->
 // update (sequential per-cluster sums in token order; also prepares the next iteration's
-// split-bf16 centres and canonical norms). The problems' heads run as four chains of launches
-// on four streams (km_fit_chains), or share every launch when no side stream is available.
+// split-bf16 centres and canonical norms). The heads of a large fit run as four chains of launches
+// on four streams (km_fit_chains); those of a small one share every launch.
 #include "base_offset.hpp"
 #include "common.hpp"
 #include "sort.hpp"
@@ -1357,7 +1357,7 @@ size_t km_workspace_bytes(int batch, int tokens, int clusters, int dims) {
     return km_workspace_raw(batch, tokens, clusters, dims) + 64 * 32;
 }
 
-// A fit runs as four chains of launches, one on the caller's stream and the others on
+// A large fit runs as four chains of launches, one on the caller's stream and the others on
 // library-owned streams of the current device (default priority), forked from the caller's
 // stream with one event and joined back to it with one event per side stream. Two layouts:
 //   - by problem: each problem's batch entries (heads) in two halves, one problem per chain.
@@ -1367,6 +1367,12 @@ size_t km_workspace_bytes(int batch, int tokens, int clusters, int dims) {
 //     takes a quarter of both problems' heads, sharing its launches (larger-K assign blocks
 //     first), so the four chains carry equal work and end together: the 480p layer 1.089-1.091
 //     against 1.104-1.111 ms by problem (fit 0.617-0.632 against 0.625-0.646 ms).
+// A fit of few workgroups is one chain of launches shared by its problems, on the caller's stream:
+// with up to kFitChainBlocks / 2 assign workgroups per CU (the problems together) the chip takes
+// them in one or two rounds anyway, and a quarter of the launches costs the host a quarter (queued /
+// alone, one chain against four; 64 + 256 centres, 10 iterations: 3 heads x 6750 tokens 343 / 391
+// against 573 / 683 us, 12 heads 509 / 555 against 555 / 773, 16 heads 556 / 602 against 559 / 793, 24
+// heads x 5000 593 / 640 against 562 / 802, the first that stays with four).
 // More chains than the process's four hardware queues serialize (the 480p fit 0.92 ms with six
 // or eight), and at 720p the layouts are within 1%. The streams and events are created once
 // per device; the mutex keeps one fork-join at a time per process on the host. If the streams
@@ -1374,6 +1380,7 @@ size_t km_workspace_bytes(int batch, int tokens, int clusters, int dims) {
 constexpr int kFitChains = 4;
 constexpr int kFitParts = 2;                    // chains per problem in the by-problem layout
 constexpr int kMixedTokens = 16384;
+constexpr int kFitChainBlocks = 7;
 constexpr int kSideStreams = kFitChains - 1;
 
 struct SideStream {
@@ -1502,7 +1509,12 @@ hipError_t km_fit_chains(const KmFitDesc* descs, int num, int dims, int dtype, i
 hipError_t km_fit(const KmFitDesc* descs, int num, int dims, int dtype, int iterations, void* workspace,
                   float* sums, hipStream_t stream) {
     bool split = !sums;  // the sums output of a one-problem fit is not sliced
-    for (int q = 0; q < num; ++q) split = split && descs[q].batch >= kFitParts;
+    int64_t blocks = 0;  // assign workgroups of an iteration
+    for (int q = 0; q < num; ++q) {
+        split = split && descs[q].batch >= kFitParts;
+        blocks += descs[q].batch * ceil_div(descs[q].tokens, kAssignTile);
+    }
+    split = split && 2 * blocks > kFitChainBlocks * static_cast<int64_t>(device_compute_units());
     if (split) {
         SideStream side[kSideStreams];
         std::mutex* m = nullptr;
