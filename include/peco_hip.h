@@ -153,6 +153,15 @@ int peco_base_offset_decode(const uint8_t* codes, const float* low, const float*
 int peco_base_offset_fake_quant(const void* x, int dtype, const int32_t* labels, const float* centroids, int batch,
                                 int tokens, int clusters, int dims, int bits, void* out, void* stream);
 
+/* The same with int32 or int64 labels (label_bytes 4 or 8). apply writes any of codes, low, scale and
+ * xhat (each nullable); reconstruct is the decoder. */
+int peco_base_offset_apply(const void* x, int dtype, const void* labels, int label_bytes, const float* centroids,
+                           int batch, int tokens, int clusters, int dims, int bits, uint8_t* codes, float* low,
+                           float* scale, void* xhat, void* stream);
+int peco_base_offset_reconstruct(const uint8_t* codes, const float* low, const float* scale, const void* labels,
+                                 int label_bytes, const float* centroids, int batch, int tokens, int clusters, int dims,
+                                 int dtype, void* out, void* stream);
+
 /* One launch packing up to 3 tensors [batch, length, dims] (fuses peco/processor.py:141-149):
  * rows [0, video) in the order of indices[i] [batch, video], fake-quantized against
  * labels[i]/centroids[i] when bits[i] is 4 or 8; rows [video, length) copied unchanged. */

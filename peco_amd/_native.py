@@ -123,6 +123,8 @@ SIGNATURES = {
     "peco_base_offset_encode": (I, [P, I, P, P, I, I, I, I, I, P, P, P, P]),
     "peco_base_offset_decode": (I, [P, P, P, P, P, I, I, I, I, I, P, P]),
     "peco_base_offset_fake_quant": (I, [P, I, P, P, I, I, I, I, I, P, P]),
+    "peco_base_offset_apply": (I, [P, I, P, I, P] + [I] * 5 + [P] * 5),
+    "peco_base_offset_reconstruct": (I, [P, P, P, P, I, P] + [I] * 5 + [P, P]),
     "peco_pack_clustered": (I, [PP, PP, PP, PP, PP, IP, IP, I, I, I, I, I, I, P]),
     "peco_sparse_attention_workspace_size": (Z, [I, I, I, I, I]),
     "peco_sparse_attention_ex": (I, [P] * 8 + [I, P, P, Z] + [I] * 7 + [P]),

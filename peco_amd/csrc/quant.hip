@@ -16,62 +16,116 @@
 namespace peco {
 namespace {
 
-template <int DT, int G>
-__global__ __launch_bounds__(256) void base_offset_kernel(const void* __restrict__ x, const int32_t* __restrict__ labels,
-                                                          const float* __restrict__ centroids, int64_t rows,
-                                                          int tokens, int clusters, int bits,
-                                                          uint8_t* __restrict__ codes, float* __restrict__ low,
-                                                          float* __restrict__ scale, void* __restrict__ xhat) {
+// Standalone quantizer and decoder. A workgroup takes kQuantPasses passes of 256 / G consecutive rows
+// of one batch entry: the labels of every pass are requested first, then the rows, then the
+// centres the labels select, so one group of lanes has four rows in flight and no thread divides a
+// 64-bit row index. With a batch divisible by the XCD count entry b runs on XCD b % kXcdCount, whose
+// L2 then fetches only its own entries' centres. 24 x 6750 x 128 bf16 rows, 4 bits: 18
+// us to encode (62 MB) or fake-quantize (83 MB, 4.6 TB/s), 14.5 to decode (4.3 TB/s); one row per
+// group and step took 20.5, 20.5 and 16.3.
+constexpr int kQuantPasses = 4;
+
+struct QuantArgs {
+    const void* x;            // encode: [batch, tokens, D]
+    const void* labels;       // [batch, tokens]
+    const float* centroids;   // [batch, clusters, D]
+    uint8_t* codes;           // encode: nullable output; decode: input
+    float* low;
+    float* scale;
+    void* xhat;               // encode: nullable
+    int batch, tokens, clusters, per_batch;
+    float levels;
+};
+
+template <typename L, int G> struct QuantRows {
+    static constexpr int R = 256 / G;
+    int b, t0, sub;
+    int64_t row0;
+    const float* cent;
+    int label[kQuantPasses];
+    __device__ __forceinline__ QuantRows(const QuantArgs& a) {
+        int chunk;
+        const int block = blockIdx.x;
+        if (a.batch % kXcdCount == 0) {
+            const int slot = block / kXcdCount;
+            b = block % kXcdCount + kXcdCount * (slot / a.per_batch);
+            chunk = slot % a.per_batch;
+        } else {
+            b = block / a.per_batch;
+            chunk = block % a.per_batch;
+        }
+        t0 = chunk * R * kQuantPasses + static_cast<int>(threadIdx.x) / G;
+        sub = threadIdx.x % G;
+        row0 = static_cast<int64_t>(b) * a.tokens;
+        cent = a.centroids + static_cast<int64_t>(b) * a.clusters * (G * 8) + sub * 8;
+#pragma unroll
+        for (int u = 0; u < kQuantPasses; ++u) {  // clamped: every load is unconditional
+            const L v = static_cast<const L*>(a.labels)[row0 + min(t0 + u * R, a.tokens - 1)];
+            // Out-of-range labels (never valid input) read the last centre instead of past the end.
+            label[u] = static_cast<int>(min(static_cast<uint64_t>(static_cast<int64_t>(v)),
+                                            static_cast<uint64_t>(a.clusters - 1)));
+        }
+    }
+    __device__ __forceinline__ int64_t at(const QuantArgs& a, int u) const { return row0 + min(t0 + u * R, a.tokens - 1); }
+    __device__ __forceinline__ bool valid(const QuantArgs& a, int u) const { return t0 + u * R < a.tokens; }
+};
+
+template <int DT, int G, typename L>
+__global__ __launch_bounds__(256) void base_offset_kernel(QuantArgs a) {
     constexpr int D = G * 8;
-    const int sub = threadIdx.x % G;
-    const float levels = static_cast<float>((1 << bits) - 1);
-    for (int64_t row = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / G; row < rows;
-         row += static_cast<int64_t>(gridDim.x) * blockDim.x / G) {
-        const int64_t b = row / tokens;
-        const int lab = labels[row];
-        float xv[8], cv[8], out[8], lo, sc;
-        uint8_t q[8];
-        Row8<DT>::load(x, row * D + sub * 8, xv);
-        load_centroid8(centroids + (b * clusters + lab) * D + sub * 8, cv);
-        base_offset_lane<G>(xv, cv, levels, out, q, lo, sc);
-        if (codes) {
+    const QuantRows<L, G> q(a);
+    float x[kQuantPasses][8], c[kQuantPasses][8];
+#pragma unroll
+    for (int u = 0; u < kQuantPasses; ++u) Row8<DT>::load(a.x, q.at(a, u) * D + q.sub * 8, x[u]);
+#pragma unroll
+    for (int u = 0; u < kQuantPasses; ++u) load_centroid8(q.cent + static_cast<int64_t>(q.label[u]) * D, c[u]);
+#pragma unroll
+    for (int u = 0; u < kQuantPasses; ++u) {
+        float out[8], lo, sc;
+        uint8_t k[8];
+        base_offset_lane<G>(x[u], c[u], a.levels, out, k, lo, sc);
+        if (!q.valid(a, u)) continue;
+        const int64_t row = q.at(a, u);
+        if (a.codes) {
             u32x2 packed;
-            packed[0] = q[0] | (q[1] << 8) | (q[2] << 16) | (static_cast<uint32_t>(q[3]) << 24);
-            packed[1] = q[4] | (q[5] << 8) | (q[6] << 16) | (static_cast<uint32_t>(q[7]) << 24);
-            *reinterpret_cast<u32x2*>(codes + row * D + sub * 8) = packed;
+            packed[0] = k[0] | (k[1] << 8) | (k[2] << 16) | (static_cast<uint32_t>(k[3]) << 24);
+            packed[1] = k[4] | (k[5] << 8) | (k[6] << 16) | (static_cast<uint32_t>(k[7]) << 24);
+            *reinterpret_cast<u32x2*>(a.codes + row * D + q.sub * 8) = packed;
         }
-        if (sub == 0) {
-            if (low) low[row] = lo;
-            if (scale) scale[row] = sc;
+        if (q.sub == 0) {
+            if (a.low) a.low[row] = lo;
+            if (a.scale) a.scale[row] = sc;
         }
-        if (xhat) Row8<DT>::store(xhat, row * D + sub * 8, out);
+        if (a.xhat) Row8<DT>::store(a.xhat, row * D + q.sub * 8, out);
     }
 }
 
-template <int DT, int G>
-__global__ __launch_bounds__(256) void base_offset_decode_kernel(const uint8_t* __restrict__ codes,
-                                                                 const float* __restrict__ low,
-                                                                 const float* __restrict__ scale,
-                                                                 const int32_t* __restrict__ labels,
-                                                                 const float* __restrict__ centroids, int64_t rows,
-                                                                 int tokens, int clusters, void* __restrict__ xhat) {
+template <int DT, int G, typename L>
+__global__ __launch_bounds__(256) void base_offset_decode_kernel(QuantArgs a) {
     constexpr int D = G * 8;
-    const int sub = threadIdx.x % G;
-    for (int64_t row = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / G; row < rows;
-         row += static_cast<int64_t>(gridDim.x) * blockDim.x / G) {
-        const int64_t b = row / tokens;
-        float cv[8], out[8];
-        load_centroid8(centroids + (b * clusters + labels[row]) * D + sub * 8, cv);
-        const u32x2 packed = *reinterpret_cast<const u32x2*>(codes + row * D + sub * 8);
-        const float lo = low[row], sc = scale[row];
+    const QuantRows<L, G> q(a);
+    u32x2 packed[kQuantPasses];
+    float lo[kQuantPasses], sc[kQuantPasses], c[kQuantPasses][8];
+#pragma unroll
+    for (int u = 0; u < kQuantPasses; ++u) {
+        packed[u] = *reinterpret_cast<const u32x2*>(a.codes + q.at(a, u) * D + q.sub * 8);
+        lo[u] = a.low[q.at(a, u)];
+        sc[u] = a.scale[q.at(a, u)];
+    }
+#pragma unroll
+    for (int u = 0; u < kQuantPasses; ++u) load_centroid8(q.cent + static_cast<int64_t>(q.label[u]) * D, c[u]);
+#pragma unroll
+    for (int u = 0; u < kQuantPasses; ++u) {
+        if (!q.valid(a, u)) continue;
+        float out[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            const uint32_t code = (packed[i / 4] >> (8 * (i % 4))) & 0xffu;
-            const float step = sc * static_cast<float>(code);
-            const float resid = lo + step;
-            out[i] = cv[i] + resid;
+            const uint32_t code = (packed[u][i / 4] >> (8 * (i % 4))) & 0xffu;
+            const float step = sc[u] * static_cast<float>(code);
+            const float resid = lo[u] + step;
+            out[i] = c[u][i] + resid;
         }
-        Row8<DT>::store(xhat, row * D + sub * 8, out);
+        Row8<DT>::store(a.xhat, q.at(a, u) * D + q.sub * 8, out);
     }
 }
 
@@ -125,36 +179,37 @@ __global__ __launch_bounds__(256) void pack_kernel(PackArgs a) {
     Row8<DT>::store(T.output, dst, out);
 }
 
-int grid_for_rows(int64_t rows, int G) {
-    const int64_t threads = rows * G;
-    return static_cast<int>(std::min<int64_t>(ceil_div(threads, 256), 1 << 20));
-}
-
-template <template <int, int> class K, typename... Args>
-bool dispatch_dt_g(int dtype, int dims, int64_t rows, hipStream_t s, Args... args) {
-#define PECO_LAUNCH(DT_, G_)                                                                             \
-    hipLaunchKernelGGL((K<DT_, G_>::kernel), dim3(grid_for_rows(rows, G_)), dim3(256), 0, s, args...); \
-    return true;
+template <bool kDecode, typename L>
+int launch_quant(QuantArgs a, int dtype, int dims, hipStream_t s) {
     const int G = dims / 8;
+    a.per_batch = static_cast<int>(ceil_div(a.tokens, 256 / G * kQuantPasses));
+    const int64_t blocks = static_cast<int64_t>(a.batch) * a.per_batch;
+    if (blocks > 0x7fffffff) return kUnsupportedShape;
+#define PECO_LAUNCH(DT_, G_)                                                                                        \
+    do {                                                                                                            \
+        if constexpr (kDecode)                                                                                      \
+            hipLaunchKernelGGL((base_offset_decode_kernel<DT_, G_, L>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, a); \
+        else                                                                                                        \
+            hipLaunchKernelGGL((base_offset_kernel<DT_, G_, L>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, a); \
+        return hipGetLastError();                                                                                   \
+    } while (0)
     if (dtype == kBF16) {
-        if (G == 16) { PECO_LAUNCH(kBF16, 16) }
-        if (G == 8) { PECO_LAUNCH(kBF16, 8) }
+        if (G == 16) PECO_LAUNCH(kBF16, 16);
+        PECO_LAUNCH(kBF16, 8);
     } else if (dtype == kF16) {
-        if (G == 16) { PECO_LAUNCH(kF16, 16) }
-        if (G == 8) { PECO_LAUNCH(kF16, 8) }
+        if (G == 16) PECO_LAUNCH(kF16, 16);
+        PECO_LAUNCH(kF16, 8);
     } else if (dtype == kF32) {
-        if (G == 16) { PECO_LAUNCH(kF32, 16) }
-        if (G == 8) { PECO_LAUNCH(kF32, 8) }
+        if (G == 16) PECO_LAUNCH(kF32, 16);
+        PECO_LAUNCH(kF32, 8);
     }
 #undef PECO_LAUNCH
-    return false;
+    return kUnsupportedDtype;
 }
 
-template <int DT, int G> struct EncodeK { static constexpr auto kernel = base_offset_kernel<DT, G>; };
-template <int DT, int G> struct DecodeK { static constexpr auto kernel = base_offset_decode_kernel<DT, G>; };
-
-bool valid_quant_args(int batch, int tokens, int clusters, int dims) {
-    return batch >= 1 && tokens >= 1 && clusters >= 1 && (dims == 64 || dims == 128);
+bool valid_quant_args(int batch, int tokens, int clusters, int dims, int label_bytes) {
+    return batch >= 1 && tokens >= 1 && clusters >= 1 && (dims == 64 || dims == 128) &&
+           (label_bytes == 4 || label_bytes == 8);
 }
 
 }  // namespace
@@ -162,42 +217,52 @@ bool valid_quant_args(int batch, int tokens, int clusters, int dims) {
 
 using namespace peco;
 
+PECO_API int peco_base_offset_apply(const void* x, int dtype, const void* labels, int label_bytes, const float* centroids,
+                                    int batch, int tokens, int clusters, int dims, int bits, uint8_t* codes, float* low,
+                                    float* scale, void* xhat, void* stream) {
+    if (!x || !labels || !centroids || !valid_quant_args(batch, tokens, clusters, dims, label_bytes) ||
+        (bits != 4 && bits != 8))
+        return kInvalidValue;
+    const QuantArgs a{x, labels, centroids, codes, low, scale, xhat, batch, tokens, clusters, 0,
+                      static_cast<float>((1 << bits) - 1)};
+    const auto s = static_cast<hipStream_t>(stream);
+    return label_bytes == 4 ? launch_quant<false, int32_t>(a, dtype, dims, s)
+                            : launch_quant<false, int64_t>(a, dtype, dims, s);
+}
+
+PECO_API int peco_base_offset_reconstruct(const uint8_t* codes, const float* low, const float* scale, const void* labels,
+                                          int label_bytes, const float* centroids, int batch, int tokens, int clusters,
+                                          int dims, int dtype, void* out, void* stream) {
+    if (!codes || !low || !scale || !labels || !centroids || !out ||
+        !valid_quant_args(batch, tokens, clusters, dims, label_bytes))
+        return kInvalidValue;
+    const QuantArgs a{nullptr, labels, centroids, const_cast<uint8_t*>(codes), const_cast<float*>(low),
+                      const_cast<float*>(scale), out, batch, tokens, clusters, 0, 0.0f};
+    const auto s = static_cast<hipStream_t>(stream);
+    return label_bytes == 4 ? launch_quant<true, int32_t>(a, dtype, dims, s)
+                            : launch_quant<true, int64_t>(a, dtype, dims, s);
+}
+
 PECO_API int peco_base_offset_encode(const void* x, int dtype, const int32_t* labels, const float* centroids,
                                      int batch, int tokens, int clusters, int dims, int bits, uint8_t* codes,
                                      float* low, float* scale, void* stream) {
-    if (!x || !labels || !centroids || !valid_quant_args(batch, tokens, clusters, dims) || (bits != 4 && bits != 8))
-        return kInvalidValue;
-    const int64_t rows = static_cast<int64_t>(batch) * tokens;
-    if (!dispatch_dt_g<EncodeK>(dtype, dims, rows, static_cast<hipStream_t>(stream), x, labels, centroids, rows,
-                                tokens, clusters, bits, codes, low, scale, static_cast<void*>(nullptr)))
-        return kUnsupportedDtype;
-    return hipGetLastError();
+    return peco_base_offset_apply(x, dtype, labels, 4, centroids, batch, tokens, clusters, dims, bits, codes, low, scale,
+                                  nullptr, stream);
 }
 
 PECO_API int peco_base_offset_decode(const uint8_t* codes, const float* low, const float* scale,
                                      const int32_t* labels, const float* centroids, int batch, int tokens,
                                      int clusters, int dims, int dtype, void* out, void* stream) {
-    if (!codes || !low || !scale || !labels || !centroids || !out || !valid_quant_args(batch, tokens, clusters, dims))
-        return kInvalidValue;
-    const int64_t rows = static_cast<int64_t>(batch) * tokens;
-    if (!dispatch_dt_g<DecodeK>(dtype, dims, rows, static_cast<hipStream_t>(stream), codes, low, scale, labels,
-                                centroids, rows, tokens, clusters, out))
-        return kUnsupportedDtype;
-    return hipGetLastError();
+    return peco_base_offset_reconstruct(codes, low, scale, labels, 4, centroids, batch, tokens, clusters, dims, dtype,
+                                        out, stream);
 }
 
 PECO_API int peco_base_offset_fake_quant(const void* x, int dtype, const int32_t* labels, const float* centroids,
                                          int batch, int tokens, int clusters, int dims, int bits, void* out,
                                          void* stream) {
-    if (!x || !labels || !centroids || !out || !valid_quant_args(batch, tokens, clusters, dims) ||
-        (bits != 4 && bits != 8))
-        return kInvalidValue;
-    const int64_t rows = static_cast<int64_t>(batch) * tokens;
-    if (!dispatch_dt_g<EncodeK>(dtype, dims, rows, static_cast<hipStream_t>(stream), x, labels, centroids, rows,
-                                tokens, clusters, bits, static_cast<uint8_t*>(nullptr), static_cast<float*>(nullptr),
-                                static_cast<float*>(nullptr), out))
-        return kUnsupportedDtype;
-    return hipGetLastError();
+    if (!out) return kInvalidValue;
+    return peco_base_offset_apply(x, dtype, labels, 4, centroids, batch, tokens, clusters, dims, bits, nullptr, nullptr,
+                                  nullptr, out, stream);
 }
 
 // One launch packs up to three tensors (Q, K, V) of shape [batch, length, dims]:

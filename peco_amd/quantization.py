@@ -51,7 +51,7 @@ def _validate_bits(bits: int, *, allow_bypass: bool) -> None:
 
 
 def _flatten_inputs(x, labels, centroids):
-    """Checks of peco/quantization.py:62-89; returns (flat x, labels int64, centroids fp32)."""
+    """Checks of peco/quantization.py:62-89; returns (flat x, labels, centroids fp32)."""
     if x.ndim not in (3, 4):
         raise ValueError("x must have shape [BH,N,D] or [B,H,N,D]")
     if any(size == 0 for size in x.shape):
@@ -74,12 +74,11 @@ def _flatten_inputs(x, labels, centroids):
         raise ValueError("HIP Base-Offset quantization supports head dimensions 64 and 128")
     if x.dtype not in _DTYPES:
         raise TypeError("x must be float16, bfloat16 or float32")
-    return flat, labels.to(torch.int64), centroids.float()
+    return flat, labels, centroids.float()
 
 
 def _launch_args(flat, labels, centroids):
-    lab32 = labels.to(torch.int32).contiguous()
-    return flat.contiguous(), lab32, centroids.contiguous()
+    return flat.contiguous(), labels.contiguous(), centroids.contiguous()
 
 
 @torch.no_grad()
@@ -87,21 +86,21 @@ def quantize_base_offset(x, labels, centroids, bits: int = 4) -> BaseOffsetQuant
     """Encode Q or K against its assigned cluster's vector centroid (bits 4 or 8)."""
     _validate_bits(bits, allow_bypass=False)
     flat, labels, centroids = _flatten_inputs(x, labels, centroids)
-    xs, lab32, cent = _launch_args(flat, labels, centroids)
+    xs, lab, cent = _launch_args(flat, labels, centroids)
     bh, n, d = xs.shape
     codes = torch.empty((bh, n, d), dtype=torch.uint8, device=xs.device)
     low = torch.empty((bh, n, 1), dtype=torch.float32, device=xs.device)
     scale = torch.empty((bh, n, 1), dtype=torch.float32, device=xs.device)
     library = _native.library()
     with torch.cuda.device(xs.device):
-        status = library.peco_base_offset_encode(
-            _native.ptr(xs), _DTYPES[xs.dtype], _native.ptr(lab32), _native.ptr(cent), bh, n, cent.shape[1], d, bits,
-            _native.ptr(codes), _native.ptr(low), _native.ptr(scale),
-            _native.current_stream(xs.device, xs, lab32, cent, codes, low, scale),
+        status = library.peco_base_offset_apply(
+            _native.ptr(xs), _DTYPES[xs.dtype], _native.ptr(lab), lab.element_size(), _native.ptr(cent), bh, n,
+            cent.shape[1], d, bits, _native.ptr(codes), _native.ptr(low), _native.ptr(scale), None,
+            _native.current_stream(xs.device, xs, lab, cent, codes, low, scale),
         )
     _native.check(status, "Base-Offset encode")
-    return BaseOffsetQuantized(centroids=centroids, labels=labels, codes=codes, offset_min=low, scale=scale,
-                               original_dtype=x.dtype, original_shape=tuple(x.shape), bits=bits)
+    return BaseOffsetQuantized(centroids=centroids, labels=labels.to(torch.int64), codes=codes, offset_min=low,
+                               scale=scale, original_dtype=x.dtype, original_shape=tuple(x.shape), bits=bits)
 
 
 @torch.no_grad()
@@ -110,16 +109,17 @@ def dequantize_base_offset(encoded: BaseOffsetQuantized) -> torch.Tensor:
     codes = encoded.codes.contiguous()
     bh, n, d = codes.shape
     cent = encoded.centroids.float().contiguous()
-    lab32 = encoded.labels.to(torch.int32).contiguous()
+    lab = encoded.labels if encoded.labels.dtype in (torch.int32, torch.int64) else encoded.labels.to(torch.int32)
+    lab = lab.contiguous()
     low = encoded.offset_min.float().contiguous()
     scale = encoded.scale.float().contiguous()
     out = torch.empty((bh, n, d), dtype=encoded.original_dtype, device=codes.device)
     library = _native.library()
     with torch.cuda.device(codes.device):
-        status = library.peco_base_offset_decode(
-            _native.ptr(codes), _native.ptr(low), _native.ptr(scale), _native.ptr(lab32), _native.ptr(cent), bh, n,
-            cent.shape[1], d, _DTYPES[encoded.original_dtype], _native.ptr(out),
-            _native.current_stream(codes.device, codes, low, scale, lab32, cent, out),
+        status = library.peco_base_offset_reconstruct(
+            _native.ptr(codes), _native.ptr(low), _native.ptr(scale), _native.ptr(lab), lab.element_size(),
+            _native.ptr(cent), bh, n, cent.shape[1], d, _DTYPES[encoded.original_dtype], _native.ptr(out),
+            _native.current_stream(codes.device, codes, low, scale, lab, cent, out),
         )
     _native.check(status, "Base-Offset decode")
     return out.reshape(encoded.original_shape)
@@ -132,14 +132,15 @@ def fake_quantize_base_offset(x, labels, centroids, bits: int = 4) -> torch.Tens
     if bits == 0:
         return x
     flat, labels, centroids = _flatten_inputs(x, labels, centroids)
-    xs, lab32, cent = _launch_args(flat, labels, centroids)
+    xs, lab, cent = _launch_args(flat, labels, centroids)
     bh, n, d = xs.shape
     out = torch.empty_like(xs)
     library = _native.library()
     with torch.cuda.device(xs.device):
-        status = library.peco_base_offset_fake_quant(
-            _native.ptr(xs), _DTYPES[xs.dtype], _native.ptr(lab32), _native.ptr(cent), bh, n, cent.shape[1], d, bits,
-            _native.ptr(out), _native.current_stream(xs.device, xs, lab32, cent, out),
+        status = library.peco_base_offset_apply(
+            _native.ptr(xs), _DTYPES[xs.dtype], _native.ptr(lab), lab.element_size(), _native.ptr(cent), bh, n,
+            cent.shape[1], d, bits, None, None, None, _native.ptr(out),
+            _native.current_stream(xs.device, xs, lab, cent, out),
         )
     _native.check(status, "Base-Offset fake quantization")
     return out.reshape(x.shape)
