@@ -1372,7 +1372,11 @@ size_t km_workspace_bytes(int batch, int tokens, int clusters, int dims) {
 // them in one or two rounds anyway, and a quarter of the launches costs the host a quarter (queued /
 // alone, one chain against four; 64 + 256 centres, 10 iterations: 3 heads x 6750 tokens 343 / 391
 // against 573 / 683 us, 12 heads 509 / 555 against 555 / 773, 16 heads 556 / 602 against 559 / 793, 24
-// heads x 5000 593 / 640 against 562 / 802, the first that stays with four).
+// heads x 5000 593 / 640 against 562 / 802, the first that stays with four). So is a fit of so few
+// iterations that the chains have nothing to run ahead of, up to kFitChainIterBlocks workgroups
+// per CU over its iterations (24 heads, 100 + 500 centres, two iterations of 6750 tokens 210 / 251
+// against 221 / 318 us, 10000 288 / 332 against 295 / 379, 16000 430 / 472 against 407 / 452; three
+// of 6750 306 / 346 against 298 / 387).
 // More chains than the process's four hardware queues serialize (the 480p fit 0.92 ms with six
 // or eight), and at 720p the layouts are within 1%. The streams and events are created once
 // per device; the mutex keeps one fork-join at a time per process on the host. If the streams
@@ -1381,6 +1385,7 @@ constexpr int kFitChains = 4;
 constexpr int kFitParts = 2;                    // chains per problem in the by-problem layout
 constexpr int kMixedTokens = 16384;
 constexpr int kFitChainBlocks = 7;
+constexpr int kFitChainIterBlocks = 16;
 constexpr int kSideStreams = kFitChains - 1;
 
 struct SideStream {
@@ -1514,7 +1519,8 @@ hipError_t km_fit(const KmFitDesc* descs, int num, int dims, int dtype, int iter
         split = split && descs[q].batch >= kFitParts;
         blocks += descs[q].batch * ceil_div(descs[q].tokens, kAssignTile);
     }
-    split = split && 2 * blocks > kFitChainBlocks * static_cast<int64_t>(device_compute_units());
+    split = split && 2 * blocks > kFitChainBlocks * static_cast<int64_t>(device_compute_units()) &&
+            iterations * blocks > kFitChainIterBlocks * static_cast<int64_t>(device_compute_units());
     if (split) {
         SideStream side[kSideStreams];
         std::mutex* m = nullptr;

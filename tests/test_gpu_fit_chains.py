@@ -30,12 +30,12 @@ def test_chained_fit_equals_each_head_alone(heads, tokens, problems, pack):
     length = tokens + 7
     sets = [_problem(g, heads, tokens, clusters, length) for clusters in (20, 70)[:problems]]
     spec = [(4, length, None)] * problems if pack else None
-    outs = clustering_cuda.kmeans_fit(sets, 3, pack=spec, pack_order="original" if pack else "cluster")
+    outs = clustering_cuda.kmeans_fit(sets, 5, pack=spec, pack_order="original" if pack else "cluster")
     packed = outs[1] if pack else None
     outs = outs[0] if pack else outs
     for i, p in enumerate(sets):
         for h in (0, heads // 4, heads // 2, heads - 1):
-            one = clustering_cuda.kmeans_fit([_head(p, h)], 3, pack=spec and spec[:1],
+            one = clustering_cuda.kmeans_fit([_head(p, h)], 5, pack=spec and spec[:1],
                                              pack_order="original" if pack else "cluster")
             fit = one[0][0] if pack else one[0]
             assert all(torch.equal(a[h], b[0]) for a, b in zip(outs[i], fit))
