@@ -291,15 +291,17 @@ size_t peco_dense_attention_workspace_size(int bh, int s);
 int peco_dense_attention(const void* q, const void* k, const void* v, void* output, int valid, int32_t* workspace,
                          size_t workspace_ints, int bh, int s, int d, int dtype, void* stream);
 
-/* Projected rows into a head-major attention buffer (peco/processor.py:159-190 after the projection
- * and norm): input [batch, heads, rows, dims] (fp16/bf16, dims 64 or 128, element strides of
+/* Projected rows into a head-major attention buffer (peco/processor.py:159-190 after the projection):
+ * input [batch, heads, rows, dims] (fp16/bf16, dims 64 or 128, element strides of
  * batch, head and row, channels adjacent, rows 16-byte aligned) is written to rows [first, first +
- * rows) of output [batch, heads, length, dims]. With cos/sin (fp32 [rows, dims], both or neither)
- * the rows are rotated over interleaved channel pairs: x * cos + (-x1, x0) * sin in fp32, rounded
- * once to the dtype. */
+ * rows) of output [batch, heads, length, dims]. With norm != 0 each row is first divided by its root
+ * mean square, 1 / sqrt(mean(x^2) + eps), and multiplied by weight [dims] (of the input's dtype, 16-byte
+ * aligned; null: ones) in fp32, rounded once to the dtype. With cos/sin (fp32 [rows, dims], both or
+ * neither) the rows are then rotated over interleaved channel pairs: x * cos + (-x1, x0) * sin in
+ * fp32, rounded once to the dtype. */
 int peco_place_heads(const void* input, int64_t stride_batch, int64_t stride_head, int64_t stride_row, void* output,
-                     const float* cos, const float* sin, int batch, int heads, int rows, int first, int length,
-                     int dims, int dtype, void* stream);
+                     const float* cos, const float* sin, int norm, const void* weight, float eps, int batch,
+                     int heads, int rows, int first, int length, int dims, int dtype, void* stream);
 
 /* peco_sparse_attention without a workspace argument. No counterpart in the reference: it is
  * for callers that cannot allocate device memory (code under HIP graph capture, serving loops

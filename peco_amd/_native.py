@@ -139,7 +139,7 @@ SIGNATURES = {
     "peco_check_cluster_sizes": (I, [P, P] + [I] * 5 + [P, P]),
     "peco_dense_attention_workspace_size": (Z, [I, I]),
     "peco_dense_attention": (I, [P] * 4 + [I, P, Z] + [I] * 4 + [P]),
-    "peco_place_heads": (I, [P] + [ctypes.c_int64] * 3 + [P] * 3 + [I] * 7 + [P]),
+    "peco_place_heads": (I, [P] + [ctypes.c_int64] * 3 + [P] * 3 + [I, P, ctypes.c_float] + [I] * 7 + [P]),
     "peco_base_offset_attention": (I, [P, P, P, I] + [P] * 9 + [I, I] + [P] * 5 + [Z] + [I] * 8 + [P]),
 }
 

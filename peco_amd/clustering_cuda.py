@@ -490,18 +490,20 @@ def pack_clustered(tensors, indices, labels, centroids, bits, video):
     return outs
 
 
-def place_heads(part, output, first, tables=None):
+def place_heads(part, output, first, tables=None, rms=None):
     """Write a projected tensor [B,H,R,D] (16-bit, any strides with adjacent channels and 16-byte
-    aligned rows) to rows [first, first + R) of the head-major output [B,H,S,D], rotated by tables =
-    (cos, sin), fp32 [R, D], over interleaved channel pairs when given (peco/processor.py:159-190)."""
+    aligned rows) to rows [first, first + R) of the head-major output [B,H,S,D], RMS-normalised over
+    the channels by rms = (weight [D] or None, eps) and rotated by tables = (cos, sin), fp32 [R, D],
+    over interleaved channel pairs when given (peco/processor.py:159-190)."""
     library = _library()
     b, h, rows, d = part.shape
     cos, sin = tables if tables is not None else (None, None)
+    weight, eps = rms if rms is not None else (None, 0.0)
     with torch.cuda.device(part.device):
         status = library.peco_place_heads(
-            _native.ptr(part), *part.stride()[:3], _native.ptr(output), _native.ptr(cos), _native.ptr(sin), b, h, rows,
-            first, output.shape[2], d, _DTYPES[part.dtype],
-            _retain_on_current_stream(part.device, part, output, cos, sin))
+            _native.ptr(part), *part.stride()[:3], _native.ptr(output), _native.ptr(cos), _native.ptr(sin),
+            int(rms is not None), _native.ptr(weight), eps, b, h, rows, first, output.shape[2], d, _DTYPES[part.dtype],
+            _retain_on_current_stream(part.device, part, output, cos, sin, weight))
     _raise_cluster_error(status)
 
 

@@ -131,6 +131,21 @@ def _per_channel_norm(norm):
         not hooks._global_forward_hooks and not hooks._global_forward_pre_hooks
 
 
+def _rms_norm(norm, part):
+    """(weight, eps) when ``norm`` is a plain RMS norm over the channels of ``part`` [B, H, rows, D]
+    that the placing kernel can apply in its place (weights of the same 16-bit dtype), else None."""
+    if type(norm) is not torch.nn.RMSNorm or not _per_channel_norm(norm) or not isinstance(norm.eps, float) or \
+            tuple(norm.normalized_shape) != (part.shape[3],) or part.dtype not in (torch.bfloat16, torch.float16) or \
+            torch.is_autocast_enabled("cuda"):
+        return None
+    weight = norm.weight
+    if weight is not None:
+        if not _native.plain_tensors(weight) or weight.dtype != part.dtype or weight.device != part.device or \
+                not weight.is_contiguous() or weight.data_ptr() % 16:
+            return None
+    return weight, norm.eps
+
+
 def _published_rotary(fn):
     return fn is _apply_rotary_emb or (getattr(fn, "__module__", "") == "diffusers.models.embeddings" and
                                        getattr(fn, "__name__", "") == "apply_rotary_emb")
@@ -150,12 +165,14 @@ def _rotary_tables(fn, freqs, rows, dim, device):
 
 
 def _placeable(part, buffer):
-    """Whether place_heads takes ``part`` [B, H, rows, D] into ``buffer`` [3, B, H, S, D]: the shapes
-    and dtype agree and its rows start on 16 bytes with adjacent channels."""
-    return part.shape[:2] == buffer.shape[1:3] and part.shape[3] == buffer.shape[4] and part.shape[3] in (64, 128) and \
-        part.shape[2] > 0 and part.dtype == buffer.dtype and part.dtype in (torch.bfloat16, torch.float16) and \
+    """Whether place_heads takes ``part`` [B, H, rows, D] into ``buffer`` [3, B, H, S, D] (None: any that
+    fits): the shapes and dtype agree and its rows start on 16 bytes with adjacent channels."""
+    if buffer is not None and (part.shape[:2] != buffer.shape[1:3] or part.shape[3] != buffer.shape[4] or
+                               part.dtype != buffer.dtype or not _native.plain_tensors(buffer)):
+        return False
+    return part.shape[3] in (64, 128) and part.shape[2] > 0 and part.dtype in (torch.bfloat16, torch.float16) and \
         part.is_cuda and part.stride(3) == 1 and all(s % 8 == 0 for s in part.stride()[:3]) and \
-        part.data_ptr() % 16 == 0 and part.shape[0] <= 65535 and _native.plain_tensors(part, buffer)
+        part.data_ptr() % 16 == 0 and part.shape[0] <= 65535 and _native.plain_tensors(part)
 
 
 class _FitResult:
@@ -341,9 +358,9 @@ class PecoAttention:
         ``attention_mask`` is ignored: which text rows are valid comes from the shared
         InferenceContext. The sequence is [video rows, text rows]. Each projection of each
         part is written once, head-major, into its slot of one [3, B, H, S, D] buffer, so no
-        concatenation copies are made; one launch per projection splits the heads, applies the
-        rotary embedding and places the rows (torch operations do it for tensors that launch does
-        not take). Video rows get the rotary embedding; text rows never do. Double-stream blocks
+        concatenation copies are made; one launch per projection splits the heads, applies a plain
+        RMS norm and the rotary embedding and places the rows (torch operations do it for tensors that
+        launch does not take). Video rows get the rotary embedding; text rows never do. Double-stream blocks
         (``add_q_proj`` set) project the text with their added projections and norms,
         single-stream blocks with the same ones as the video.
         """
@@ -365,22 +382,24 @@ class PecoAttention:
             rows = source.shape[1]
             for slot, proj in enumerate(projections):
                 part = proj(source).unflatten(2, (attn.heads, -1)).transpose(1, 2)  # [B, H, rows, D] view
-                tables = None
-                if slot < 2:
-                    if norms[slot] is not None:
-                        # The rows as projected, where the norm cannot tell: no copy into head order first.
-                        swap = part.is_cuda and _per_channel_norm(norms[slot])
-                        part = norms[slot](part.transpose(1, 2)).transpose(1, 2) if swap else norms[slot](part)
-                    if freqs is not None:
-                        tables = _rotary_tables(rotary, freqs, rows, part.shape[3], part.device)
-                        if tables is None:
-                            part = rotary(part, freqs)
+                norm = norms[slot] if slot < 2 else None
+                turn = slot < 2 and freqs is not None
+                tables = _rotary_tables(rotary, freqs, rows, part.shape[3], part.device) if turn else None
+                turn = turn and tables is None  # by torch
+                rms = None if norm is None or turn or not _placeable(part, None) else _rms_norm(norm, part)
+                if norm is not None and rms is None:
+                    # The rows as projected, where the norm cannot tell: no copy into head order first.
+                    swap = part.is_cuda and _per_channel_norm(norm)
+                    part = norm(part.transpose(1, 2)).transpose(1, 2) if swap else norm(part)
+                if turn:
+                    part = rotary(part, freqs)
                 if qkv is None:
                     batch, heads, _, dim = part.shape
                     qkv = torch.empty((3, batch, heads, length, dim), dtype=part.dtype, device=part.device)
                 if _placeable(part, qkv):
-                    clustering_cuda.place_heads(part, qkv[slot], first, tables)
+                    clustering_cuda.place_heads(part, qkv[slot], first, tables, rms)
                 else:
+                    part = part if rms is None else norm(part)
                     qkv[slot, :, :, first:first + rows] = part if tables is None else rotary(part, freqs)
             first += rows
         output = self.attention(qkv[0], qkv[1], qkv[2]).transpose(1, 2)  # [B, S, H, D] view

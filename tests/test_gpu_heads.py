@@ -35,6 +35,36 @@ def test_place_heads_matches_torch(dtype, dim, batch, heads, rows, first, length
             assert torch.equal(out.nan_to_num(3.0), ref.nan_to_num(3.0))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("batch,heads,rows,first,length", [
+    (1, 1, 1, 0, 1), (1, 7, 15, 3, 20), (2, 8, 16, 0, 16), (1, 9, 17, 5, 40), (1, 24, 333, 0, 400)])
+def test_place_heads_rms_norm(dtype, dim, batch, heads, rows, first, length):
+    """Bound: the fp32 sum of squares (at most 9 roundings on the way of a term), eps, the inverse root
+    (one ulp) and two products are within 20 * 2^-24 of the real value, then one rounding to the dtype
+    (2^-8 or 2^-11, and half the smallest fp16 subnormal)."""
+    g = torch.Generator().manual_seed(rows * heads + dim)
+    x = (torch.randn(batch, rows, heads, dim, generator=g) * 3.0).to(dtype).to(DEV)
+    x[0, 0, 0] = 0.0
+    weight = (1.0 + torch.rand(dim, generator=g)).to(dtype).to(DEV)
+    tables = _tables(rows, dim, g)
+    for part in (x.transpose(1, 2), x.transpose(1, 2).contiguous()):
+        for w in (weight, None):
+            out = torch.full((batch, heads, length, dim), 7.0, dtype=dtype, device=DEV)
+            clustering_cuda.place_heads(part, out, first, None, (w, 1e-6))
+            wide = part.double()
+            ref = wide / (wide.square().mean(-1, keepdim=True) + 1e-6).sqrt() * (1.0 if w is None else w.double())
+            placed = out[:, :, first:first + rows]
+            unit = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+            assert ((placed.double() - ref).abs() <= (unit + 20 * 2.0 ** -24) * 1.01 * ref.abs() + 2.0 ** -25).all()
+            module = torch.nn.functional.rms_norm(part.transpose(1, 2), (dim,), w, 1e-6).transpose(1, 2)
+            assert torch.equal(placed, module)
+            assert (out[:, :, :first] == 7.0).all() and (out[:, :, first + rows:] == 7.0).all()
+            turned = torch.empty_like(out)
+            clustering_cuda.place_heads(part, turned, first, tables, (w, 1e-6))
+            assert torch.equal(turned[:, :, first:first + rows], processor._apply_rotary_emb(placed, tables))
+
+
 class _Block(torch.nn.Module):
     def __init__(self, heads, dim, double):
         super().__init__()
