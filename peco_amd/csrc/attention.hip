@@ -1502,8 +1502,9 @@ namespace {
 
 // Work list of the two groups, one workgroup per head: per group one key segment, items of `tile`
 // rows in row order (all of a group cost alike, the valid rows' group first), zeroed queues.
-__global__ __launch_bounds__(256) void build_dense_kernel(int32_t* ws, int bhn, int s, int valid, int tile) {
-    const SelWork W = sel_work_layout(ws, bhn, s, 2, 2);
+__global__ __launch_bounds__(256) void build_dense_kernel(int32_t* ws, int bhn, int s, int valid, int tile,
+                                                          int layout_rows) {
+    const SelWork W = sel_work_layout(ws, bhn, layout_rows, 2, 2);
     const int bh = blockIdx.x, tid = threadIdx.x;
     const int n0 = static_cast<int>(ceil_div(valid, tile)), n1 = static_cast<int>(ceil_div(s - valid, tile));
     int32_t* items = W.items + static_cast<int64_t>(bh) * W.cap * 3;
@@ -1527,18 +1528,26 @@ __global__ __launch_bounds__(256) void build_dense_kernel(int32_t* ws, int bhn, 
 
 // Rows per item: full 256-row items on 8-wavefront workgroups when they still fill the CUs twice
 // (every K/V tile then serves twice the rows: 11.8 against 12.3 ms at 24 heads x 32896 rows, 0.62
-// against 0.63 ms at 7006), else 128-row items, which spread a short call over more CUs.
+// against 0.63 ms at 7006), else 128-row items, which spread a short call over more CUs, or 64-row
+// items when all of those run at once: their waves pair up and split the keys of a tile, so each
+// item, and with it the launch, is shorter (128 channels, 128- against 64-row items: 3 heads x 1024
+// rows 33 and 24 us, 8 x 2100 58 and 42, 3 x 7006 159 and 136, 2 x 16000 337 and 312).
+constexpr int kDenseShort = 64;
 int dense_item_rows(int bh, int s) {
-    return static_cast<int64_t>(bh) * (s / (2 * kQTile)) >= 2 * static_cast<int64_t>(device_compute_units()) ? 2 * kQTile
-                                                                                                           : kQTile;
+    const int64_t slots = 2 * static_cast<int64_t>(device_compute_units());
+    if (static_cast<int64_t>(bh) * (s / (2 * kQTile)) >= slots) return 2 * kQTile;
+    return bh * (ceil_div(s, kDenseShort) + 1) <= slots ? kDenseShort : kQTile;
 }
+
+// Query rows the work list is laid out for: its capacity counts items of kQTile rows.
+int dense_layout_rows(int tile, int s) { return tile < kQTile ? s * (kQTile / tile) : s; }
 
 }  // namespace
 }  // namespace peco
 
 PECO_API size_t peco_dense_attention_workspace_size(int bh, int s) {
     if (bh < 1 || s < 0) return 0;
-    return sel_work_ints(bh, s, 2, 2);
+    return sel_work_ints(bh, dense_layout_rows(dense_item_rows(bh, s), s), 2, 2);
 }
 
 PECO_API int peco_dense_attention(const void* q, const void* k, const void* v, void* output, int valid, int32_t* workspace,
@@ -1547,11 +1556,11 @@ PECO_API int peco_dense_attention(const void* q, const void* k, const void* v, v
         (d != 64 && d != 128) || (dtype != kF16 && dtype != kBF16))
         return kInvalidValue;
     if (s == 0) return kOk;
-    if (workspace_ints < sel_work_ints(bh, s, 2, 2)) return kWorkspaceTooSmall;
+    const int tile = dense_item_rows(bh, s), rows = dense_layout_rows(tile, s);
+    if (workspace_ints < sel_work_ints(bh, rows, 2, 2)) return kWorkspaceTooSmall;
     const auto st = static_cast<hipStream_t>(stream);
-    const int tile = dense_item_rows(bh, s);
-    hipLaunchKernelGGL(build_dense_kernel, dim3(bh), dim3(256), 0, st, workspace, bh, s, valid, tile);
-    const SelWork W = sel_work_layout(workspace, bh, s, 2, 2);
+    hipLaunchKernelGGL(build_dense_kernel, dim3(bh), dim3(256), 0, st, workspace, bh, s, valid, tile, rows);
+    const SelWork W = sel_work_layout(workspace, bh, rows, 2, 2);
     return launch_attention_kernel(q, k, v, nullptr, nullptr, W.segs, W.counts, W.items, W.cap, output, nullptr, 0,
                                    nullptr, nullptr, 0, 0, bh, s, s, d, 2, 2, dtype, W.queues, tile, 0.0f, st);
 }

@@ -44,6 +44,16 @@ def test_dense_attention_matches_reference(dtype, batch, heads, length, dim, val
         assert err.max().item() <= 2e-2 and err.mean().item() <= 2e-3
 
 
+@pytest.mark.parametrize("heads,length,dim,valid", [
+    (64, 448, 128, 383), (64, 449, 64, 320), (128, 192, 64, 129), (3, 1025, 128, 1024), (2, 4097, 64, 65)])
+def test_dense_attention_short_items(heads, length, dim, valid):
+    """64-row items while all of them run at once (448 and 192 rows are the last such lengths of their
+    head counts, 449 takes 128-row items), with items of 64 rows, of one row and past a whole tile."""
+    q, k, v = _inputs(1, heads, length, dim, torch.bfloat16)
+    err = (processor.dense_attention(q, k, v, valid).float() - _reference(q, k, v, valid)).abs()
+    assert err.max().item() <= 2e-2 and err.mean().item() <= 2e-3
+
+
 def test_dense_attention_keeps_layout_and_sdpa_calls():
     q, k, v = (t.transpose(1, 2).contiguous().transpose(1, 2) for t in _inputs(1, 4, 200, 64, torch.bfloat16))
     out = processor.dense_attention(q, k, v, 150)
