@@ -335,7 +335,7 @@ __device__ __forceinline__ void attention_item(
     const int32_t* __restrict__ counts, const int32_t* __restrict__ items, int cap, uint16_t* __restrict__ out,
     const int32_t* __restrict__ out_index, int oi_rows, const int32_t* __restrict__ k_index,
     const float* __restrict__ qcent, int qcent_rows, float levels, int bhn, int band, int sq, int sk, int cq,
-    int ck, float scale_log2, float lazy) {
+    int ck, float scale_log2, float lazy, int pair_rows) {
     constexpr bool kIndexedKV = kMode == kIndexed || kMode == kIndexedQuantQ;
     constexpr bool kQuantLoad = kMode == kQuantQ || kMode == kIndexedQuantQ;
     using T = Tiles<D>;
@@ -376,11 +376,11 @@ __device__ __forceinline__ void attention_item(
     const int64_t head = static_cast<int64_t>(bh);
     const uint32_t sq_last = static_cast<uint32_t>(sq - 1), sk_last = static_cast<uint32_t>(sk - 1);
 
-    // Items of at most 32 * H rows pair the waves: wave w takes 32-row block w % H and, of
-    // every tile, only the 32-key half w / H, so a short item's tiles cost about half the
+    // Items of at most pair_rows <= 32 * H rows pair the waves: wave w takes 32-row block w % H
+    // and, of every tile, only the 32-key half w / H, so a short item's tiles cost about half the
     // time; each pair merges its two partial softmax states after the last tile. Longer items
     // give each wave its own row block and both halves of every tile.
-    const bool split = q_rows <= 32 * H;
+    const bool split = q_rows <= pair_rows;
     const int rb = split ? (wave % H) : wave;  // this wave's 32-row block
     const int hb = split ? (wave / H) : 0;     // first 32-key half this wave processes
     // Waves without query rows issue every tile load, so that waiting for the load path to
@@ -815,11 +815,11 @@ __global__ __launch_bounds__(kWaves * kWave, 8 / kWaves) void sparse_attention_k
     const int32_t* __restrict__ counts, const int32_t* __restrict__ items, int cap, uint16_t* __restrict__ out,
     const int32_t* __restrict__ out_index, int oi_rows, const int32_t* __restrict__ k_index,
     const float* __restrict__ qcent, int qcent_rows, float levels, int bhn, int band, int sq, int sk, int cq,
-    int ck, float scale_log2, float lazy, int32_t* __restrict__ queues, int nwg) {
+    int ck, float scale_log2, float lazy, int pair_rows, int32_t* __restrict__ queues, int nwg) {
     if constexpr (!kPersist) {
         attention_item<DT, D, kMode, kWaves>(blockIdx.x, q, k, v, selected, kprefix, segs, counts, items, cap, out,
                                              out_index, oi_rows, k_index, qcent, qcent_rows, levels, bhn, band, sq,
-                                             sk, cq, ck, scale_log2, lazy);
+                                             sk, cq, ck, scale_log2, lazy, pair_rows);
     } else {
         __shared__ int next;
         const int total = cap * bhn;
@@ -836,7 +836,7 @@ __global__ __launch_bounds__(kWaves * kWave, 8 / kWaves) void sparse_attention_k
             x = g % kItemQueues;
             attention_item<DT, D, kMode, kWaves>(g, q, k, v, selected, kprefix, segs, counts, items, cap, out,
                                                  out_index, oi_rows, k_index, qcent, qcent_rows, levels, bhn, band, sq,
-                                                 sk, cq, ck, scale_log2, lazy);
+                                                 sk, cq, ck, scale_log2, lazy, pair_rows);
         }
         if (threadIdx.x == 0 && atomicAdd(&queues[kItemQueues], 1) == nwg - 1) {
             for (int x = 0; x <= kItemQueues; ++x)
@@ -1326,6 +1326,18 @@ int attention_head_band(int bh, int sk, int d) {
     return 1;
 }
 
+// How the items of a work list run: `rows` as the list was cut, on workgroups of `waves` wavefronts (8,
+// one per CU, or 4, two per CU), items of at most pair_rows <= 16 * waves rows with paired waves.
+struct ItemForm {
+    int rows;
+    int waves;
+    int pair_rows;
+};
+ItemForm sparse_item_form(int sq) {
+    const int rows = attention_item_rows(sq), waves = rows == 2 * kQTile ? 8 : 4;
+    return {rows, waves, 16 * waves};
+}
+
 // Launch of the attention kernel over a built work list (map + kprefix, or segs).
 // q_centroids (nullable, with out_index) selects the kQuantQ input mode, or kIndexedQuantQ
 // with k_index.
@@ -1343,7 +1355,7 @@ int launch_attention_kernel(const void* q, const void* k, const void* v, const u
                             const int32_t* kprefix, const int2* segs, const int32_t* counts, const int32_t* items,
                             int cap, void* output, const int32_t* out_index, int out_index_rows,
                             const int32_t* k_index, const float* q_centroids, int q_clusters, int bits, int bh,
-                            int sq, int sk, int d, int cq, int ck, int dtype, int32_t* queues, int item_rows,
+                            int sq, int sk, int d, int cq, int ck, int dtype, int32_t* queues, ItemForm form,
                             float lazy_log2, hipStream_t s) {
     const int mode = k_index ? (q_centroids ? kIndexedQuantQ : kIndexed) : (q_centroids ? kQuantQ : kPacked);
     const float levels = static_cast<float>((1 << bits) - 1);
@@ -1351,9 +1363,7 @@ int launch_attention_kernel(const void* q, const void* k, const void* v, const u
     const float scale_log2 = static_cast<float>(1.4426950408889634 / std::sqrt(static_cast<double>(d)));
     const float lazy = lazy_log2 / scale_log2;  // in units of the raw scores
     const int64_t total = static_cast<int64_t>(cap) * bh;
-    // Items of 2 * kQTile rows (item_rows, as the work list was cut) run on 8-wavefront
-    // workgroups, one per CU; others on 4-wavefront ones, two per CU.
-    const int waves = item_rows == 2 * kQTile ? 8 : 4;
+    const int waves = form.waves;
     const int nwg = static_cast<int>(
         std::min<int64_t>(total, (8 / waves) * static_cast<int64_t>(device_compute_units())));
     if (queues && total < static_cast<int64_t>(kPersistItems) * nwg) queues = nullptr;
@@ -1366,7 +1376,7 @@ int launch_attention_kernel(const void* q, const void* k, const void* v, const u
 #define PECO_ATTN_P(DT_, D_, M_, P_, W_)                                                                           \
     hipLaunchKernelGGL((sparse_attention_kernel<DT_, D_, M_, P_, W_>), grid, dim3(W_ * kWave), lds_attn, s, qp, kp, \
                        vp, selected, kprefix, segs, counts, items, cap, op, out_index, out_index_rows, k_index,      \
-                       q_centroids, q_clusters, levels, bh, band, sq, sk, cq, ck, scale_log2, lazy, queues, nwg)
+                       q_centroids, q_clusters, levels, bh, band, sq, sk, cq, ck, scale_log2, lazy, form.pair_rows, queues, nwg)
 #define PECO_ATTN(DT_, D_, M_, W_)                                                                                 \
     do {                                                                                                           \
         if (queues) PECO_ATTN_P(DT_, D_, M_, true, W_);                                                            \
@@ -1426,7 +1436,7 @@ int launch_sparse_attention(const void* q, const void* k, const void* v, const u
     const WorkLayout W = work_layout(workspace, bh, sq, cq, ck);
     return launch_attention_kernel(q, k, v, selected, W.kprefix, nullptr, W.counts, W.items, W.cap, output, out_index,
                                    out_index_rows, k_index, nullptr, 0, 0, bh, sq, sk, d, cq, ck, dtype, nullptr,
-                                   attention_item_rows(sq), kLazyLog2, s);
+                                   sparse_item_form(sq), kLazyLog2, s);
 }
 
 }  // namespace
@@ -1487,33 +1497,42 @@ PECO_API int peco_sparse_attention_work(const void* q, const void* k, const void
     return launch_attention_kernel(q, k, v, nullptr, nullptr, W.segs, W.counts, W.items, W.cap, output, out_index,
                                    out_index_rows, k_index, q_centroids, q_centroids ? q_clusters : 0,
                                    q_centroids ? bits : 0, bh, sq, sk, d, cq, ck, dtype, W.queues,
-                                   attention_item_rows(sq), kLazyLog2, static_cast<hipStream_t>(stream));
+                                   sparse_item_form(sq), kLazyLog2, static_cast<hipStream_t>(stream));
 }
 
 // Dense attention of a warm-up step (peco/processor.py:52-65): rows [0, valid) attend to each other
 // and so do rows [valid, s), as two row groups of the work list above. MFMA-bound: full items over
-// one long key segment. Library SDPA, which needs each segment sliced into contiguous copies, took
-// 21.9 ms for 24 heads x 32896 rows x 128 channels in bf16 (609 TFLOP/s) and 1.64 ms at 7006 rows;
-// here 12.5 ms (1067 TFLOP/s; large bf16 matrix products reach 1190-1250 on this card) and 0.71
-// ms. O is rescaled at every new row maximum (see lazy_log2): with the sparse calls' lazy
-// threshold the error against 64 bits was 10% above SDPA's on peaked rows.
+// one long key segment. In bf16 with 128 channels, 24 heads x 32896 rows take 12.3 ms (1076 TFLOP/s;
+// large bf16 matrix products reach 1190-1250 on this card) and 24 x 7006 rows 0.64 ms; library SDPA,
+// which needs each segment sliced into contiguous copies, took 21.9 and 1.63 ms. O is rescaled at
+// every new row maximum (see lazy_log2): with the sparse calls' lazy threshold the error against
+// 64 bits was 10% above SDPA's on peaked rows.
 namespace peco {
 namespace {
 
+constexpr int kDenseShort = 64;  // rows of the paired items
+
 // Work list of the two groups, one workgroup per head: per group one key segment, items of `tile`
-// rows in row order (all of a group cost alike, the valid rows' group first), zeroed queues.
+// rows in row order (all of a group cost alike, the valid rows' group first), zeroed queues. Items of at
+// most kDenseShort rows pair their waves, so a group's last rows % kQTile rows, when they are that few,
+// are an item of their own whatever `tile` is.
 __global__ __launch_bounds__(256) void build_dense_kernel(int32_t* ws, int bhn, int s, int valid, int tile,
                                                           int layout_rows) {
     const SelWork W = sel_work_layout(ws, bhn, layout_rows, 2, 2);
     const int bh = blockIdx.x, tid = threadIdx.x;
-    const int n0 = static_cast<int>(ceil_div(valid, tile)), n1 = static_cast<int>(ceil_div(s - valid, tile));
     int32_t* items = W.items + static_cast<int64_t>(bh) * W.cap * 3;
-    for (int i = tid; i < n0 + n1; i += blockDim.x) {
-        const int g = i >= n0;
-        const int begin = (g ? valid : 0) + (g ? i - n0 : i) * tile;
-        items[3 * i + 0] = begin;
-        items[3 * i + 1] = g;
-        items[3 * i + 2] = min(tile, (g ? s : valid) - begin);
+    int count = 0;
+    for (int g = 0; g < 2; ++g) {
+        const int rows = g ? s - valid : valid, tail = rows % kQTile;
+        const int body = tail <= kDenseShort ? rows - tail : rows;  // rows of the items before such a one
+        const int n = static_cast<int>(ceil_div(body, tile)), n1 = n + static_cast<int>(ceil_div(rows - body, tile));
+        for (int i = tid; i < n1; i += blockDim.x) {
+            const int begin = i < n ? i * tile : body + (i - n) * tile;
+            items[3 * (count + i) + 0] = (g ? valid : 0) + begin;
+            items[3 * (count + i) + 1] = g;
+            items[3 * (count + i) + 2] = min(tile, (i < n ? body : rows) - begin);
+        }
+        count += n1;
     }
     if (tid < 2) {
         const int rows = tid ? s - valid : valid;
@@ -1522,21 +1541,33 @@ __global__ __launch_bounds__(256) void build_dense_kernel(int32_t* ws, int bhn, 
         seg[1] = rows > 0 ? int2{tid ? valid : 0, 0} : int2{0, 0x7fffffff};
         seg[2] = int2{0, 0x7fffffff};
     }
-    if (tid == 0) W.counts[bh] = n0 + n1;
+    if (tid == 0) W.counts[bh] = count;
     if (bh == 0 && tid < kQueueInts) W.queues[tid] = 0;
 }
 
-// Rows per item: full 256-row items on 8-wavefront workgroups when they still fill the CUs twice
-// (every K/V tile then serves twice the rows: 11.8 against 12.3 ms at 24 heads x 32896 rows, 0.62
-// against 0.63 ms at 7006), else 128-row items, which spread a short call over more CUs, or 64-row
-// items when all of those run at once: their waves pair up and split the keys of a tile, so each
-// item, and with it the launch, is shorter (128 channels, 128- against 64-row items: 3 heads x 1024
-// rows 33 and 24 us, 8 x 2100 58 and 42, 3 x 7006 159 and 136, 2 x 16000 337 and 312).
-constexpr int kDenseShort = 64;
-int dense_item_rows(int bh, int s) {
+// A head's output must not depend on how many heads share its call. Paired waves keep a softmax state
+// per half of every key tile, which rounds differently from unpaired ones, so whether a row's item pairs
+// follows from the length and the channels alone; between unpaired items of 128 and 256 rows no bit
+// differs, and the head count may choose.
+// - Up to kDensePairElems elements of K per head: 64-row items, all paired. They spread a call of few
+//   heads over twice the CUs; with many heads they read every tile twice as often. us, against the
+//   better unpaired form, for 3 / 12 / 24 heads: 128 channels, 1024 rows 23 / 24 / 31 against 32 / 32 /
+//   32, 4096 rows (the line) 69 / 156 / 257 against 100 / 135 / 242, 7006 rows 138 / 404 / 772 against
+//   159 / 370 / 645; 64 channels, 4096 rows 49 / 83 / 151 against 72 / 98 / 134, 7006 rows 99 / 235 / 413
+//   against 114 / 207 / 394, 12000 rows 196 / 579 / 1312 against 248 / 560 / 985.
+// - Above: with 128 channels 256-row items on 8-wavefront workgroups when they fill the CUs twice (every
+//   K/V tile then serves twice the rows: 24 heads x 32896 rows 12.3 against 12.6 ms, x 7006 0.64
+//   against 0.67), else 128-row items; with 64 channels always 128-row items, whose 4-wavefront
+//   workgroups fit more than two to a CU there (24 heads x 12000 rows 985 against 1215 us, x 32896 7.7
+//   against 8.3 ms).
+constexpr int64_t kDensePairElems = int64_t{1} << 19;
+bool dense_pairs(int s, int d) { return static_cast<int64_t>(s) * d <= kDensePairElems; }
+
+ItemForm dense_item_form(int bh, int s, int d) {
+    if (dense_pairs(s, d)) return {kDenseShort, 4, kDenseShort};
     const int64_t slots = 2 * static_cast<int64_t>(device_compute_units());
-    if (static_cast<int64_t>(bh) * (s / (2 * kQTile)) >= slots) return 2 * kQTile;
-    return bh * (ceil_div(s, kDenseShort) + 1) <= slots ? kDenseShort : kQTile;
+    if (d == 128 && static_cast<int64_t>(bh) * (s / (2 * kQTile)) >= slots) return {2 * kQTile, 8, kDenseShort};
+    return {kQTile, 4, kDenseShort};
 }
 
 // Query rows the work list is laid out for: its capacity counts items of kQTile rows.
@@ -1547,7 +1578,8 @@ int dense_layout_rows(int tile, int s) { return tile < kQTile ? s * (kQTile / ti
 
 PECO_API size_t peco_dense_attention_workspace_size(int bh, int s) {
     if (bh < 1 || s < 0) return 0;
-    return sel_work_ints(bh, dense_layout_rows(dense_item_rows(bh, s), s), 2, 2);
+    // Enough for either channel count: the shortest items the length can take.
+    return sel_work_ints(bh, dense_layout_rows(dense_pairs(s, 64) ? kDenseShort : kQTile, s), 2, 2);
 }
 
 PECO_API int peco_dense_attention(const void* q, const void* k, const void* v, void* output, int valid, int32_t* workspace,
@@ -1556,13 +1588,14 @@ PECO_API int peco_dense_attention(const void* q, const void* k, const void* v, v
         (d != 64 && d != 128) || (dtype != kF16 && dtype != kBF16))
         return kInvalidValue;
     if (s == 0) return kOk;
-    const int tile = dense_item_rows(bh, s), rows = dense_layout_rows(tile, s);
+    const ItemForm form = dense_item_form(bh, s, d);
+    const int rows = dense_layout_rows(form.rows, s);
     if (workspace_ints < sel_work_ints(bh, rows, 2, 2)) return kWorkspaceTooSmall;
     const auto st = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(build_dense_kernel, dim3(bh), dim3(256), 0, st, workspace, bh, s, valid, tile, rows);
+    hipLaunchKernelGGL(build_dense_kernel, dim3(bh), dim3(256), 0, st, workspace, bh, s, valid, form.rows, rows);
     const SelWork W = sel_work_layout(workspace, bh, rows, 2, 2);
     return launch_attention_kernel(q, k, v, nullptr, nullptr, W.segs, W.counts, W.items, W.cap, output, nullptr, 0,
-                                   nullptr, nullptr, 0, 0, bh, s, s, d, 2, 2, dtype, W.queues, tile, 0.0f, st);
+                                   nullptr, nullptr, 0, 0, bh, s, s, d, 2, 2, dtype, W.queues, form, 0.0f, st);
 }
 
 // Base-Offset integer-score attention (an extension with no counterpart in the reference; see

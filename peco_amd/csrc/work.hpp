@@ -24,14 +24,16 @@ constexpr int kItemBits = 12;  // sort payload: query cluster (high bits), item 
 // serves twice the query rows, halving the tile loads per row (their clusters mostly exceed 128
 // rows). Measured: the 720p attention (119056 rows) 1.7% faster, the 544p one (32896 rows) 1.3%
 // slower, where one workgroup per CU hides less of the loads' latency than two. The
-// work-list builders and the attention launch use this one rule, which depends on the query
-// length alone, so a work list always meets the workgroups it was cut for.
+// work-list builders and the launch of the sparse attention use this one rule, which depends on
+// the query length alone, so a work list always meets the workgroups it was cut for. (The dense
+// list has a rule of its own, dense_item_form in attention.hip.)
 constexpr int kLongItemsFrom = 65536;
 __host__ __device__ inline int attention_item_rows(int sq) {
     return sq >= kLongItemsFrom ? 2 * kQTile : kQTile;
 }
 
-// Item slots per head: enough for items of kQTile rows (longer items need fewer).
+// Item slots per head: enough for items of kQTile rows (longer items need fewer; a list of shorter
+// ones is laid out for as many more query rows).
 __host__ __device__ inline int item_capacity(int sq, int cq) {
     return static_cast<int>(ceil_div(sq, kQTile)) + min(cq, sq);
 }
@@ -41,7 +43,8 @@ __host__ __device__ inline int item_capacity(int sq, int cq) {
 //         call on a buffer, and every call leaves them zero;
 //   counts int32 [bh]: items per head;
 //   row_keys int32 [bh, re]: the stream length L of every map row;
-//   items int32 [bh, cap, 3]: q_start, query cluster, rows (<= kQTile), by descending cost;
+//   items int32 [bh, cap, 3]: q_start, query cluster, rows (at most those of the rule the list was
+//         cut by, up to 2 * kQTile), by descending cost;
 //   queues int32 [kQueueInts]: the attention's item queue counters (one per XCD) and its exit
 //         counter; zero before the first call, and every attention call leaves them zero;
 //   segs  int2 [bh, re, ce + 2] (8-byte aligned): per map row {segment count n, L}, then n

@@ -31,9 +31,12 @@ def _inputs(batch, heads, length, dim, dtype):
 @pytest.mark.parametrize("batch,heads,length,dim,valid", [
     (1, 1, 1, 128, 1), (1, 2, 63, 64, 0), (1, 2, 64, 128, 64), (2, 3, 65, 128, 64), (1, 3, 129, 64, 1),
     (1, 2, 257, 128, 128), (1, 2, 1000, 128, 937),
-    (1, 64, 2309, 64, 2100),    # 256-row items on 8-wavefront workgroups
-    (1, 64, 4300, 128, 4250),   # the same on the persistent grid
-    (10, 200, 70, 64, 40),      # 128-row items on the persistent grid
+    (1, 64, 2309, 64, 2100),    # paired 64-row items, more than run at once
+    (1, 64, 4300, 128, 4250),   # 256-row items on 8-wavefront workgroups, on the persistent grid
+    (1, 32, 4300, 128, 4113),   # the same without it
+    (1, 2, 4097, 128, 4096),    # 128-row items
+    (1, 62, 8193, 64, 8192),    # the same on the persistent grid
+    (10, 200, 70, 64, 40),      # 64-row items on the persistent grid
 ])
 def test_dense_attention_matches_reference(dtype, batch, heads, length, dim, valid):
     q, k, v = _inputs(batch, heads, length, dim, dtype)
@@ -47,8 +50,7 @@ def test_dense_attention_matches_reference(dtype, batch, heads, length, dim, val
 @pytest.mark.parametrize("heads,length,dim,valid", [
     (64, 448, 128, 383), (64, 449, 64, 320), (128, 192, 64, 129), (3, 1025, 128, 1024), (2, 4097, 64, 65)])
 def test_dense_attention_short_items(heads, length, dim, valid):
-    """64-row items while all of them run at once (448 and 192 rows are the last such lengths of their
-    head counts, 449 takes 128-row items), with items of 64 rows, of one row and past a whole tile."""
+    """Items of 64 rows, of one row and past a whole tile, few and many per head."""
     q, k, v = _inputs(1, heads, length, dim, torch.bfloat16)
     err = (processor.dense_attention(q, k, v, valid).float() - _reference(q, k, v, valid)).abs()
     assert err.max().item() <= 2e-2 and err.mean().item() <= 2e-3
@@ -76,3 +78,22 @@ def test_dense_attention_padding_segment_sees_no_video_value():
     out = processor.dense_attention(q, k, v, 250)
     assert torch.isfinite(out[0, 0, 250:]).all() and torch.isfinite(out[0, 1]).all()
     assert not torch.isfinite(out[0, 0, :250]).any()
+
+
+@pytest.mark.parametrize("length,dim,valid", [
+    (300, 128, 211), (2100, 128, 1975), (4096, 128, 4000), (4097, 128, 4000), (7006, 128, 6881),
+    (7006, 128, 6817), (7006, 128, 6693), (3000, 64, 2900),
+    (8192, 64, 8100), (8193, 64, 8100)])
+def test_dense_attention_of_a_head_is_the_same_in_any_call(length, dim, valid):
+    """A head's output does not depend on how many heads share its call: 24 heads together, as batch
+    entries and in shards of one to twelve give the same bits (lengths on both sides of the rules for
+    items)."""
+    q, k, v = _inputs(1, 24, length, dim, torch.bfloat16)
+    out = processor.dense_attention(q, k, v, valid)
+    assert torch.equal(out, processor.dense_attention(q, k, v, valid))
+    assert torch.equal(out, processor.dense_attention(*(t.view(4, 6, length, dim) for t in (q, k, v)), valid).view_as(out))
+    for a, b in ((0, 1), (21, 24), (3, 9), (12, 24)):
+        part = processor.dense_attention(*(t[:, a:b].contiguous() for t in (q, k, v)), valid)
+        assert torch.equal(part, out[:, a:b]), (a, b)
+    wide = [torch.cat((t, t, t, t), 1) for t in (q, k, v)]
+    assert torch.equal(processor.dense_attention(*wide, valid)[:, 48:72], out)
