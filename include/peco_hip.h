@@ -285,7 +285,7 @@ int peco_base_offset_attention(const void* q, const int32_t* out_index, const fl
 
 /* Dense attention of a warm-up step (peco/processor.py:52-65) on the sparse kernel's MFMA path: of
  * q/k/v [bh, s, d] (fp16/bf16, d 64 or 128), rows [0, valid) attend to each other and so do rows
- * [valid, s). workspace: peco_dense_attention_workspace_size int32 (8-byte aligned, need not be
+ * [valid, s). Tensors 16-byte aligned. workspace: peco_dense_attention_workspace_size int32 (8-byte aligned, need not be
  * cleared). */
 size_t peco_dense_attention_workspace_size(int bh, int s);
 int peco_dense_attention(const void* q, const void* k, const void* v, void* output, int valid, int32_t* workspace,

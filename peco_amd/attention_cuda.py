@@ -275,7 +275,8 @@ def dense_supported(q, k, v, valid_length) -> bool:
         1 <= q.shape[0] * q.shape[1] <= 65535 and q.dtype in (torch.float16, torch.bfloat16) and \
         q.dtype == k.dtype == v.dtype and q.is_cuda and q.device == k.device == v.device and \
         not (torch.is_grad_enabled() and any(t.requires_grad for t in (q, k, v))) and \
-        not torch.is_autocast_enabled("cuda") and _native.plain_tensors(q, k, v) and _device_is_gfx950(q.device)
+        not torch.is_autocast_enabled("cuda") and _native.plain_tensors(q, k, v) and \
+        all(t.data_ptr() % 16 == 0 or not t.is_contiguous() for t in (q, k, v)) and _device_is_gfx950(q.device)
 
 
 def dense_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, valid_length: int) -> torch.Tensor:

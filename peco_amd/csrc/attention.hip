@@ -1587,6 +1587,9 @@ PECO_API int peco_dense_attention(const void* q, const void* k, const void* v, v
     if (!q || !k || !v || !output || !workspace || bh < 1 || bh > 65535 || s < 0 || valid < 0 || valid > s ||
         (d != 64 && d != 128) || (dtype != kF16 && dtype != kBF16))
         return kInvalidValue;
+    // Rows are read and tiles loaded to LDS 16 bytes at a time.
+    for (const void* p : {q, k, v, static_cast<const void*>(output)})
+        if (reinterpret_cast<uintptr_t>(p) % 16) return kInvalidValue;
     if (s == 0) return kOk;
     const ItemForm form = dense_item_form(bh, s, d);
     const int rows = dense_layout_rows(form.rows, s);

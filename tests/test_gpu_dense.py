@@ -5,7 +5,7 @@ are those of the attention tests (P and the output are rounded to 16 bits)."""
 import pytest
 import torch
 
-from peco_amd import attention_cuda, processor
+from peco_amd import _native, attention_cuda, processor
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -97,3 +97,29 @@ def test_dense_attention_of_a_head_is_the_same_in_any_call(length, dim, valid):
         assert torch.equal(part, out[:, a:b]), (a, b)
     wide = [torch.cat((t, t, t, t), 1) for t in (q, k, v)]
     assert torch.equal(processor.dense_attention(*wide, valid)[:, 48:72], out)
+
+
+def test_dense_attention_leaves_misaligned_tensors_to_sdpa():
+    """A contiguous view that does not start on 16 bytes is not taken (the kernel loads 16 bytes at a
+    time); a strided one is copied first, wherever it starts. The C entry refuses such a pointer."""
+    aligned = _inputs(1, 2, 200, 64, torch.bfloat16)
+    ref = _reference(*aligned, 150)
+    for i in range(3):
+        views = list(aligned)
+        flat = torch.empty(views[i].numel() + 1, dtype=torch.bfloat16, device=DEV)
+        views[i] = flat[1:].view(views[i].shape).copy_(views[i])
+        assert views[i].is_contiguous() and not attention_cuda.dense_supported(*views, 150)
+        assert (processor.dense_attention(*views, 150).float() - ref).abs().max().item() <= 2e-2
+        wide = torch.empty(1, 2, 200, 65, dtype=torch.bfloat16, device=DEV)
+        views[i] = wide[..., 1:].copy_(aligned[i])
+        assert attention_cuda.dense_supported(*views, 150)
+        assert torch.equal(processor.dense_attention(*views, 150), processor.dense_attention(*aligned, 150))
+    library = _native.library()
+    ints = library.peco_dense_attention_workspace_size(2, 200)
+    workspace = torch.empty(ints, dtype=torch.int32, device=DEV)
+    out = torch.empty_like(aligned[0])
+    pointers = [t.data_ptr() for t in (*aligned, out)]
+    for i in range(4):
+        shifted = [p + 2 * (j == i) for j, p in enumerate(pointers)]
+        assert library.peco_dense_attention(*shifted, 150, _native.ptr(workspace), ints, 2, 200, 64, 1,
+                                            _native.current_stream(out.device, out)) != 0
