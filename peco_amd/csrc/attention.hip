@@ -33,6 +33,7 @@
 #include "work.hpp"
 
 #include <algorithm>
+#include <cfloat>
 #include <mutex>
 #include <type_traits>
 
@@ -320,11 +321,20 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 //     qcent[bh, qc] and levels = 2^bits - 1 (peco/processor.py:141, fused into the load);
 //   kIndexedQuantQ: Q as in kQuantQ, K and V in original order read through k_index as in
 //     kIndexed (the Base-Offset layer: K fake-quantized in original order by the fit, V the
-//     caller's own tensor).
+//     caller's own tensor);
+//   kDense: inputs as in kPacked, the two row groups of a warm-up step (peco_dense_attention).
 // The key stream of an item comes either from a kept-segment list (segs, as the selection
 // launch writes it: {count n, stream length L}, n segments, sentinel per map row) or, when segs
 // is null, from the item's map row and the clamped key-cluster prefix kprefix [bh, ck + 1].
-enum InputMode : int { kPacked = 0, kIndexed = 1, kQuantQ = 2, kIndexedQuantQ = 3 };
+enum InputMode : int { kPacked = 0, kIndexed = 1, kQuantQ = 2, kIndexedQuantQ = 3, kDense = 4 };
+
+constexpr int kDenseShort = 64;  // rows of kDense's paired items
+
+// A key's weight is exp2(fma(score, scale, -max * scale)): the fma rounds once, but -max * scale was
+// rounded before, by up to 2^-24 of itself, in the exponent of every weight of the row. That factor
+// cancels until it overflows, so kDense, which takes any scores an ordinary softmax takes, subtracts the
+// maximum first once a row's scaled maximum of the wavefront passes 2^20.
+constexpr float kWideLog2 = 0x1p20f;
 
 // One work item (linear index g over bands x slots x heads, see below) of the attention, run
 // by a workgroup of kWaves wavefronts (4, or 8 for the items of 2 * kQTile rows).
@@ -335,12 +345,16 @@ __device__ __forceinline__ void attention_item(
     const int32_t* __restrict__ counts, const int32_t* __restrict__ items, int cap, uint16_t* __restrict__ out,
     const int32_t* __restrict__ out_index, int oi_rows, const int32_t* __restrict__ k_index,
     const float* __restrict__ qcent, int qcent_rows, float levels, int bhn, int band, int sq, int sk, int cq,
-    int ck, float scale_log2, float lazy, int pair_rows) {
+    int ck, float scale_log2) {
     constexpr bool kIndexedKV = kMode == kIndexed || kMode == kIndexedQuantQ;
     constexpr bool kQuantLoad = kMode == kQuantQ || kMode == kIndexedQuantQ;
     using T = Tiles<D>;
     constexpr int S = D / 16;       // k-steps of S^T over channels
     constexpr int NB = D / 32;      // 32-channel blocks of O^T
+    // Scores may run up to 2^8 above the running maximum before O is rescaled (rescaling at every
+    // new maximum costs the sparse calls a few percent). kDense rescales at every one, so that the largest
+    // weight of a row is 1 when P is rounded to 16 bits, as in an exact softmax.
+    constexpr float kLazyLog2 = kMode == kDense ? 0.0f : 8.0f;
     // K tiles (buffers 0, 1) and V tiles (2, 3) in one array: after the last tile the paired
     // waves exchange their softmax states through it, which takes more than the K half.
     constexpr int NT = kWaves * kWave;           // threads of the workgroup
@@ -376,11 +390,13 @@ __device__ __forceinline__ void attention_item(
     const int64_t head = static_cast<int64_t>(bh);
     const uint32_t sq_last = static_cast<uint32_t>(sq - 1), sk_last = static_cast<uint32_t>(sk - 1);
 
-    // Items of at most pair_rows <= 32 * H rows pair the waves: wave w takes 32-row block w % H
-    // and, of every tile, only the 32-key half w / H, so a short item's tiles cost about half the
-    // time; each pair merges its two partial softmax states after the last tile. Longer items
+    // Items of at most 32 * H rows (kDense: kDenseShort) pair the waves: wave w takes 32-row block
+    // w % H and, of every tile, only the 32-key half w / H, so a short item's tiles cost about half
+    // the time; each pair merges its two partial softmax states after the last tile. Longer items
     // give each wave its own row block and both halves of every tile.
-    const bool split = q_rows <= pair_rows;
+    constexpr int kPairRows = kMode == kDense ? kDenseShort : 32 * H;
+    static_assert(kPairRows <= 32 * H, "paired items have at most H row blocks");
+    const bool split = q_rows <= kPairRows;
     const int rb = split ? (wave % H) : wave;  // this wave's 32-row block
     const int hb = split ? (wave / H) : 0;     // first 32-key half this wave processes
     // Waves without query rows issue every tile load, so that waiting for the load path to
@@ -519,7 +535,11 @@ __device__ __forceinline__ void attention_item(
     f32x16 oacc[NB];
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) oacc[nb] = f32x16{};
-    float m_run = -INFINITY, l_run = 0.0f, neg_m = 0.0f;
+    // kDense starts at the lowest finite value, so that a row whose scores so far are all -inf is
+    // rescaled by exp2(0) with its neighbours.
+    float m_run = kMode == kDense ? -FLT_MAX : -INFINITY, l_run = 0.0f, neg_m = 0.0f;
+    bool wide = false;
+    const float lazy = kLazyLog2 / scale_log2;
 
     const uint16_t* kh = k + head * sk * D;
     const uint16_t* vh = v + head * sk * D;
@@ -603,11 +623,21 @@ __device__ __forceinline__ void attention_item(
                 const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * scale_log2);
                 m_run = m_new;
                 neg_m = -m_new * scale_log2;
+                if constexpr (kMode == kDense) {
+                    wide = __any(fabsf(neg_m) > kWideLog2);
+                    if (wide) neg_m = 0.0f;
+                }
                 l_run *= alpha;
 #pragma unroll
                 for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
                     for (int i = 0; i < 16; ++i) oacc[nb][i] *= alpha;
+            }
+            if constexpr (kMode == kDense) {
+                if (wide) {
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) sacc[j][i] -= m_run;
+                }
             }
             uint32_t pp[8];
 #pragma unroll
@@ -740,7 +770,8 @@ __device__ __forceinline__ void attention_item(
             if (turn && hb == 0 && wave_active) {
                 const float m1 = xch[NB * 16], l1 = xch[NB * 16 + 1];
                 const float m = fmaxf(m_run, m1);
-                // A half without keys has m = -inf (and l = 0, O = 0); both empty leaves O at 0.
+                // A half without keys has m = -inf (kDense: -FLT_MAX) and l = 0, O = 0; both empty
+                // leaves O at 0.
                 const float a0 = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m_run - m) * scale_log2);
                 const float a1 = m1 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m1 - m) * scale_log2);
                 l_run = l_run * a0 + l1 * a1;
@@ -815,11 +846,11 @@ __global__ __launch_bounds__(kWaves * kWave, 8 / kWaves) void sparse_attention_k
     const int32_t* __restrict__ counts, const int32_t* __restrict__ items, int cap, uint16_t* __restrict__ out,
     const int32_t* __restrict__ out_index, int oi_rows, const int32_t* __restrict__ k_index,
     const float* __restrict__ qcent, int qcent_rows, float levels, int bhn, int band, int sq, int sk, int cq,
-    int ck, float scale_log2, float lazy, int pair_rows, int32_t* __restrict__ queues, int nwg) {
+    int ck, float scale_log2, int32_t* __restrict__ queues, int nwg) {
     if constexpr (!kPersist) {
         attention_item<DT, D, kMode, kWaves>(blockIdx.x, q, k, v, selected, kprefix, segs, counts, items, cap, out,
                                              out_index, oi_rows, k_index, qcent, qcent_rows, levels, bhn, band, sq,
-                                             sk, cq, ck, scale_log2, lazy, pair_rows);
+                                             sk, cq, ck, scale_log2);
     } else {
         __shared__ int next;
         const int total = cap * bhn;
@@ -836,7 +867,7 @@ __global__ __launch_bounds__(kWaves * kWave, 8 / kWaves) void sparse_attention_k
             x = g % kItemQueues;
             attention_item<DT, D, kMode, kWaves>(g, q, k, v, selected, kprefix, segs, counts, items, cap, out,
                                                  out_index, oi_rows, k_index, qcent, qcent_rows, levels, bhn, band, sq,
-                                                 sk, cq, ck, scale_log2, lazy, pair_rows);
+                                                 sk, cq, ck, scale_log2);
         }
         if (threadIdx.x == 0 && atomicAdd(&queues[kItemQueues], 1) == nwg - 1) {
             for (int x = 0; x <= kItemQueues; ++x)
@@ -1326,18 +1357,6 @@ int attention_head_band(int bh, int sk, int d) {
     return 1;
 }
 
-// How the items of a work list run: `rows` as the list was cut, on workgroups of `waves` wavefronts (8,
-// one per CU, or 4, two per CU), items of at most pair_rows <= 16 * waves rows with paired waves.
-struct ItemForm {
-    int rows;
-    int waves;
-    int pair_rows;
-};
-ItemForm sparse_item_form(int sq) {
-    const int rows = attention_item_rows(sq), waves = rows == 2 * kQTile ? 8 : 4;
-    return {rows, waves, 16 * waves};
-}
-
 // Launch of the attention kernel over a built work list (map + kprefix, or segs).
 // q_centroids (nullable, with out_index) selects the kQuantQ input mode, or kIndexedQuantQ
 // with k_index.
@@ -1346,24 +1365,22 @@ ItemForm sparse_item_form(int sq) {
 // sparse_attention_kernel (two resident workgroups per CU take items from the queues): 544p
 // attention 5.4% and 720p 4.2% faster than one workgroup per item, while at 480p (5.6 slots
 // per workgroup, items of about 100 us) taking each item costs more than it saves (+2.3%).
-// lazy_log2: scores may run up to 2^lazy_log2 above the running maximum before O is rescaled. The
-// sparse calls use kLazyLog2 (rescaling at every new maximum costs a few percent); 0 keeps the
-// largest weight of a row at exactly 1 when P is rounded to 16 bits, as an exact softmax does.
-constexpr float kLazyLog2 = 8.0f;
+// item_rows: rows per item, as the work list was cut. dense: the kDense mode.
 constexpr int kPersistItems = 8;
 int launch_attention_kernel(const void* q, const void* k, const void* v, const uint8_t* selected,
                             const int32_t* kprefix, const int2* segs, const int32_t* counts, const int32_t* items,
                             int cap, void* output, const int32_t* out_index, int out_index_rows,
                             const int32_t* k_index, const float* q_centroids, int q_clusters, int bits, int bh,
-                            int sq, int sk, int d, int cq, int ck, int dtype, int32_t* queues, ItemForm form,
-                            float lazy_log2, hipStream_t s) {
-    const int mode = k_index ? (q_centroids ? kIndexedQuantQ : kIndexed) : (q_centroids ? kQuantQ : kPacked);
+                            int sq, int sk, int d, int cq, int ck, int dtype, int32_t* queues, int item_rows,
+                            bool dense, hipStream_t s) {
+    const int mode = dense ? kDense : k_index ? (q_centroids ? kIndexedQuantQ : kIndexed) : (q_centroids ? kQuantQ : kPacked);
     const float levels = static_cast<float>((1 << bits) - 1);
     const size_t lds_attn = sizeof(int) * 2 * (static_cast<size_t>(ck) + 1);
     const float scale_log2 = static_cast<float>(1.4426950408889634 / std::sqrt(static_cast<double>(d)));
-    const float lazy = lazy_log2 / scale_log2;  // in units of the raw scores
     const int64_t total = static_cast<int64_t>(cap) * bh;
-    const int waves = form.waves;
+    // Items of 2 * kQTile rows run on 8-wavefront workgroups, one per CU; others on 4-wavefront ones,
+    // two per CU.
+    const int waves = item_rows == 2 * kQTile ? 8 : 4;
     const int nwg = static_cast<int>(
         std::min<int64_t>(total, (8 / waves) * static_cast<int64_t>(device_compute_units())));
     if (queues && total < static_cast<int64_t>(kPersistItems) * nwg) queues = nullptr;
@@ -1376,7 +1393,7 @@ int launch_attention_kernel(const void* q, const void* k, const void* v, const u
 #define PECO_ATTN_P(DT_, D_, M_, P_, W_)                                                                           \
     hipLaunchKernelGGL((sparse_attention_kernel<DT_, D_, M_, P_, W_>), grid, dim3(W_ * kWave), lds_attn, s, qp, kp, \
                        vp, selected, kprefix, segs, counts, items, cap, op, out_index, out_index_rows, k_index,      \
-                       q_centroids, q_clusters, levels, bh, band, sq, sk, cq, ck, scale_log2, lazy, form.pair_rows, queues, nwg)
+                       q_centroids, q_clusters, levels, bh, band, sq, sk, cq, ck, scale_log2, queues, nwg)
 #define PECO_ATTN(DT_, D_, M_, W_)                                                                                 \
     do {                                                                                                           \
         if (queues) PECO_ATTN_P(DT_, D_, M_, true, W_);                                                            \
@@ -1397,6 +1414,8 @@ int launch_attention_kernel(const void* q, const void* k, const void* v, const u
         if (mode == kIndexed) PECO_ATTN_D(DT_, kIndexed);                                                          \
         else if (mode == kQuantQ) PECO_ATTN_D(DT_, kQuantQ);                                                       \
         else if (mode == kIndexedQuantQ) PECO_ATTN_D(DT_, kIndexedQuantQ);                                         \
+        else if (mode == kDense && d == 64) PECO_ATTN(DT_, 64, kDense, 4);                                         \
+        else if (mode == kDense) PECO_ATTN_W(DT_, 128, kDense);                                                    \
         else PECO_ATTN_D(DT_, kPacked);                                                                            \
     } while (0)
     if (dtype == kBF16) PECO_ATTN_M(kBF16);
@@ -1436,7 +1455,7 @@ int launch_sparse_attention(const void* q, const void* k, const void* v, const u
     const WorkLayout W = work_layout(workspace, bh, sq, cq, ck);
     return launch_attention_kernel(q, k, v, selected, W.kprefix, nullptr, W.counts, W.items, W.cap, output, out_index,
                                    out_index_rows, k_index, nullptr, 0, 0, bh, sq, sk, d, cq, ck, dtype, nullptr,
-                                   sparse_item_form(sq), kLazyLog2, s);
+                                   attention_item_rows(sq), false, s);
 }
 
 }  // namespace
@@ -1497,7 +1516,7 @@ PECO_API int peco_sparse_attention_work(const void* q, const void* k, const void
     return launch_attention_kernel(q, k, v, nullptr, nullptr, W.segs, W.counts, W.items, W.cap, output, out_index,
                                    out_index_rows, k_index, q_centroids, q_centroids ? q_clusters : 0,
                                    q_centroids ? bits : 0, bh, sq, sk, d, cq, ck, dtype, W.queues,
-                                   sparse_item_form(sq), kLazyLog2, static_cast<hipStream_t>(stream));
+                                   attention_item_rows(sq), false, static_cast<hipStream_t>(stream));
 }
 
 // Dense attention of a warm-up step (peco/processor.py:52-65): rows [0, valid) attend to each other
@@ -1505,12 +1524,10 @@ PECO_API int peco_sparse_attention_work(const void* q, const void* k, const void
 // one long key segment. In bf16 with 128 channels, 24 heads x 32896 rows take 12.3 ms (1076 TFLOP/s;
 // large bf16 matrix products reach 1190-1250 on this card) and 24 x 7006 rows 0.64 ms; library SDPA,
 // which needs each segment sliced into contiguous copies, took 21.9 and 1.63 ms. O is rescaled at
-// every new row maximum (see lazy_log2): with the sparse calls' lazy threshold the error against
+// every new row maximum (kLazyLog2): with the sparse calls' lazy threshold the error against
 // 64 bits was 10% above SDPA's on peaked rows.
 namespace peco {
 namespace {
-
-constexpr int kDenseShort = 64;  // rows of the paired items
 
 // Work list of the two groups, one workgroup per head: per group one key segment, items of `tile`
 // rows in row order (all of a group cost alike, the valid rows' group first), zeroed queues. Items of at
@@ -1563,11 +1580,10 @@ __global__ __launch_bounds__(256) void build_dense_kernel(int32_t* ws, int bhn, 
 constexpr int64_t kDensePairElems = int64_t{1} << 19;
 bool dense_pairs(int s, int d) { return static_cast<int64_t>(s) * d <= kDensePairElems; }
 
-ItemForm dense_item_form(int bh, int s, int d) {
-    if (dense_pairs(s, d)) return {kDenseShort, 4, kDenseShort};
+int dense_item_rows(int bh, int s, int d) {
+    if (dense_pairs(s, d)) return kDenseShort;
     const int64_t slots = 2 * static_cast<int64_t>(device_compute_units());
-    if (d == 128 && static_cast<int64_t>(bh) * (s / (2 * kQTile)) >= slots) return {2 * kQTile, 8, kDenseShort};
-    return {kQTile, 4, kDenseShort};
+    return d == 128 && static_cast<int64_t>(bh) * (s / (2 * kQTile)) >= slots ? 2 * kQTile : kQTile;
 }
 
 // Query rows the work list is laid out for: its capacity counts items of kQTile rows.
@@ -1591,14 +1607,13 @@ PECO_API int peco_dense_attention(const void* q, const void* k, const void* v, v
     for (const void* p : {q, k, v, static_cast<const void*>(output)})
         if (reinterpret_cast<uintptr_t>(p) % 16) return kInvalidValue;
     if (s == 0) return kOk;
-    const ItemForm form = dense_item_form(bh, s, d);
-    const int rows = dense_layout_rows(form.rows, s);
+    const int tile = dense_item_rows(bh, s, d), rows = dense_layout_rows(tile, s);
     if (workspace_ints < sel_work_ints(bh, rows, 2, 2)) return kWorkspaceTooSmall;
     const auto st = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(build_dense_kernel, dim3(bh), dim3(256), 0, st, workspace, bh, s, valid, form.rows, rows);
+    hipLaunchKernelGGL(build_dense_kernel, dim3(bh), dim3(256), 0, st, workspace, bh, s, valid, tile, rows);
     const SelWork W = sel_work_layout(workspace, bh, rows, 2, 2);
     return launch_attention_kernel(q, k, v, nullptr, nullptr, W.segs, W.counts, W.items, W.cap, output, nullptr, 0,
-                                   nullptr, nullptr, 0, 0, bh, s, s, d, 2, 2, dtype, W.queues, form, 0.0f, st);
+                                   nullptr, nullptr, 0, 0, bh, s, s, d, 2, 2, dtype, W.queues, tile, true, st);
 }
 
 // Base-Offset integer-score attention (an extension with no counterpart in the reference; see

@@ -26,7 +26,7 @@ constexpr int kItemBits = 12;  // sort payload: query cluster (high bits), item 
 // slower, where one workgroup per CU hides less of the loads' latency than two. The
 // work-list builders and the launch of the sparse attention use this one rule, which depends on
 // the query length alone, so a work list always meets the workgroups it was cut for. (The dense
-// list has a rule of its own, dense_item_form in attention.hip.)
+// list has a rule of its own, dense_item_rows in attention.hip.)
 constexpr int kLongItemsFrom = 65536;
 __host__ __device__ inline int attention_item_rows(int sq) {
     return sq >= kLongItemsFrom ? 2 * kQTile : kQTile;

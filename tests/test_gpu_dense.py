@@ -123,3 +123,35 @@ def test_dense_attention_leaves_misaligned_tensors_to_sdpa():
         shifted = [p + 2 * (j == i) for j, p in enumerate(pointers)]
         assert library.peco_dense_attention(*shifted, 150, _native.ptr(workspace), ints, 2, 200, 64, 1,
                                             _native.current_stream(out.device, out)) != 0
+
+
+@pytest.mark.parametrize("length,dim", [(300, 64), (300, 128), (4500, 128)])
+def test_dense_attention_with_scores_of_any_size(length, dim):
+    """Large scores (on both sides of the point where a row's maximum is subtracted first) and keys with
+    scores of -inf give what an ordinary softmax gives. Rows whose two best scores differ by less than
+    the products' rounding are left out."""
+    valid = length - 50
+    plain = _inputs(1, 2, length, dim, torch.bfloat16)
+    for a, b in ((60.0, 1e3), (3e2, 4e3), (1e5, 1e5), (1e18, 1e18)):
+        q, k, v = plain[0] * a, plain[1] * b, plain[2]
+        got = processor.dense_attention(q, k, v, valid).float()
+        assert torch.isfinite(got).all()
+        for lo, hi in ((0, valid), (valid, length)):
+            scores = q[:, :, lo:hi].double() @ k[:, :, lo:hi].double().transpose(2, 3).contiguous() * dim ** -0.5
+            ref = torch.softmax(scores, -1) @ v[:, :, lo:hi].double()
+            best = scores.topk(2, -1).values
+            clear = (best[..., 0] - best[..., 1]) > 1e-5 * scores.abs().amax(-1) + 10
+            assert clear.float().mean() > 0.5
+            assert ((got[:, :, lo:hi] - ref).abs().amax(-1)[clear] <= 2e-2).all()
+    for rows in (32, 64, length):  # the first keys; every key
+        q, k, v = plain[0], plain[1].clone(), plain[2]
+        k[:, :, :rows, 0] = -float("inf")
+        got = processor.dense_attention(q, k, v, length).float()
+        none = q[..., 0] < 0  # scores of +inf: not a number
+        assert (got.isnan().all(-1) == none).all()
+        if rows < length:
+            ref = torch.softmax(q.float() @ k[:, :, rows:].float().transpose(2, 3).contiguous() * dim ** -0.5, -1) @ \
+                v[:, :, rows:].float()
+            assert ((got - ref).abs().amax(-1)[~none] <= 2e-2).all()
+        else:
+            assert (got[~none] == 0).all()  # no weight at all
