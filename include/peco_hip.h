@@ -295,7 +295,7 @@ int peco_dense_attention(const void* q, const void* k, const void* v, void* outp
  * input [batch, heads, rows, dims] (fp16/bf16, dims 64 or 128, element strides of
  * batch, head and row, channels adjacent, rows 16-byte aligned) is written to rows [first, first +
  * rows) of output [batch, heads, length, dims]. With norm != 0 each row is first divided by its root
- * mean square, 1 / sqrt(mean(x^2) + eps), and multiplied by weight [dims] (of the input's dtype, 16-byte
+ * mean square, 1 / sqrt(mean(x^2) + eps) (a subnormal sum under the root counts as 0), and multiplied by weight [dims] (of the input's dtype, 16-byte
  * aligned; null: ones) in fp32, rounded once to the dtype. With cos/sin (fp32 [rows, dims], both or
  * neither) the rows are then rotated over interleaved channel pairs: x * cos + (-x1, x0) * sin in
  * fp32, rounded once to the dtype. */

@@ -133,8 +133,10 @@ def _per_channel_norm(norm):
 
 def _rms_norm(norm, part):
     """(weight, eps) when ``norm`` is a plain RMS norm over the channels of ``part`` [B, H, rows, D]
-    that the placing kernel can apply in its place (weights of the same 16-bit dtype), else None."""
+    that the placing kernel can apply in its place (weights of the same 16-bit dtype; an eps that keeps
+    mean + eps a normal fp32 number, since the kernel's inverse root takes a subnormal one as 0), else None."""
     if type(norm) is not torch.nn.RMSNorm or not _per_channel_norm(norm) or not isinstance(norm.eps, float) or \
+            not norm.eps >= 2.0 ** -126 or \
             tuple(norm.normalized_shape) != (part.shape[3],) or part.dtype not in (torch.bfloat16, torch.float16) or \
             torch.is_autocast_enabled("cuda"):
         return None

@@ -100,3 +100,24 @@ def test_call_matches_the_torch_prologue(double, text, monkeypatch):
     ref = layer(block, hidden, enc, image_rotary_emb=freqs)
     assert torch.equal(got[0], ref[0])
     assert (got[1] is None and ref[1] is None) if not text else torch.equal(got[1], ref[1])
+
+
+@pytest.mark.parametrize("eps,size", [(0.0, 1e-20), (0.0, 3e-19), (1e-40, 1e-20), (2.0 ** -126, 1e-20), (1e-6, 1.0)])
+def test_call_with_a_norm_of_tiny_rows(eps, size):
+    """Rows whose mean square is subnormal come out as the block's norm gives them, whatever its eps."""
+    heads, dim, video = 3, 64, 40
+    torch.manual_seed(6)
+    block = _Block(heads, dim, False).to(DEV, torch.bfloat16)
+    for name in ("q", "k"):
+        norm, proj = getattr(block, "norm_" + name), getattr(block, "to_" + name)
+        norm.eps = eps
+        proj.weight.data *= size
+        proj.bias.data *= size
+    hidden = torch.randn(1, video, heads * dim, device=DEV).bfloat16()
+    layer = processor.PecoAttention(0, processor.PecoConfig(), processor.InferenceContext(5, 0, 0))
+    layer.attention = lambda q, k, v: torch.cat((q, k), -1)
+    got = layer(block, hidden, None)[0].unflatten(2, (heads, -1))
+    for at, name in ((0, "q"), (dim, "k")):
+        rows = getattr(block, "to_" + name)(hidden).unflatten(2, (heads, -1))
+        want = getattr(block, "norm_" + name)(rows)
+        assert torch.isfinite(want).all() and torch.equal(got[..., at:at + dim], want)
