@@ -102,8 +102,8 @@ int peco_kmeans_fit(int num_problems, const void* const* x, const int64_t* x_bat
 
 /* Iterations [first, first + iterations) of a one-problem fit that stops once no centre moves further
  * than tol (peco/clustering.py:61-86). Means of iteration i go to centers_a (i even) or centers_b
- * (i odd); flags int32 [iterations + 1, 1 + batch], zeroed but for row 0: all 1 when first is 0,
- * else the last row of the call before. Row t + 1 receives {1 if a centre moved past tol, per
+ * (i odd); flags int32 [iterations + 1, 1 + batch], zeroed but for row 0, which is the last row of
+ * the call before (not read when first is 0). Row t + 1 receives {1 if a centre moved past tol, per
  * entry 1 if a centre changed} of iteration first + t; after a row whose first value stays 0 the
  * later iterations change nothing (labels, counts, permutation and centres are that iteration's).
  * The workspace (peco_kmeans_workspace_size) carries the fit between calls. */
@@ -295,10 +295,10 @@ int peco_dense_attention(const void* q, const void* k, const void* v, void* outp
  * input [batch, heads, rows, dims] (fp16/bf16, dims 64 or 128, element strides of
  * batch, head and row, channels adjacent, rows 16-byte aligned) is written to rows [first, first +
  * rows) of output [batch, heads, length, dims]. With norm != 0 each row is first divided by its root
- * mean square, 1 / sqrt(mean(x^2) + eps) (a subnormal sum under the root counts as 0), and multiplied by weight [dims] (of the input's dtype, 16-byte
- * aligned; null: ones) in fp32, rounded once to the dtype. With cos/sin (fp32 [rows, dims], both or
- * neither) the rows are then rotated over interleaved channel pairs: x * cos + (-x1, x0) * sin in
- * fp32, rounded once to the dtype. */
+ * mean square, 1 / sqrt(mean(x^2) + eps) (a subnormal sum under the root counts as 0), and multiplied
+ * by weight [dims] (of the input's dtype, 16-byte aligned; null: ones) in fp32, rounded once to the
+ * dtype. With cos/sin (fp32 [rows, dims], both or neither) the rows are then rotated over
+ * interleaved channel pairs: x * cos + (-x1, x0) * sin in fp32, rounded once to the dtype. */
 int peco_place_heads(const void* input, int64_t stride_batch, int64_t stride_head, int64_t stride_row, void* output,
                      const float* cos, const float* sin, int norm, const void* weight, float eps, int batch,
                      int heads, int rows, int first, int length, int dims, int dtype, void* stream);

@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import collections
 import ctypes
+import itertools
 
 import torch
 
@@ -255,10 +256,17 @@ def kmeans_fit(problems, iterations, pack=None, pack_order="cluster"):
     return outs, packed
 
 
-# Iterations of a converging fit launched between two looks at its flags: a look costs a host
-# synchronization (about 20 us with the launches behind it, half an iteration of the 480p features),
-# launches past the stop return at once.
+# Iterations of a converging fit launched before its first looks at the flags and between the later ones.
+# A look costs about 25 us (the copy to the host, then the launches behind it), an iteration launched
+# past the stop 7-10 us (its launches return at once): a fit that starts at its fixed point, or near
+# it, should stop almost at once, a long one look rarely. us, 24 x 6750 x 128 fp32 rows in 100 centres,
+# stopping after 1 / 2 / 5 / 9 / 17 iterations: 136 / 207 / 356 / 561 / 1038; looks after 1, 3, 7, 15
+# and so on 133 / 234 / 384 / 590 / 1067; every eight 183 / 254 / 356 / 570 / 1054; a fit call and a
+# check per iteration 136 / 262 / 639 / 1141 / 2166. One entry of 500 tokens, after 1: 73, every eight 135,
+# stepwise 78.
+_TOL_FIRST = (2, 4)
 _TOL_STEP = 8
+_TOL_ROWS = 64  # rows of the flags allocated at once
 
 
 def _float32_floor(value):
@@ -283,20 +291,25 @@ def kmeans_fit_until(problem, max_iters, tol):
     offsets = torch.empty((p.batch, p.clusters + 1), dtype=torch.int32, device=dev)
     ws_bytes = library.peco_kmeans_workspace_size(p.batch, p.tokens, p.clusters, dims)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-    done, last = 0, None
+    tol = _float32_floor(tol)
+    steps = itertools.chain(_TOL_FIRST, itertools.repeat(_TOL_STEP))
+    done, flags, at = 0, None, 0
     while done < max_iters:
-        step = min(_TOL_STEP, max_iters - done)
-        flags = torch.zeros((step + 1, 1 + p.batch), dtype=torch.int32, device=dev)
-        flags[0].fill_(1) if last is None else flags[0].copy_(last)
+        step = min(next(steps), max_iters - done)
+        if flags is None or at + step >= flags.shape[0]:
+            last = None if flags is None else flags[at]
+            flags, at = torch.zeros((min(_TOL_ROWS, max_iters - done) + 1, 1 + p.batch), dtype=torch.int32, device=dev), 0
+            if last is not None:
+                flags[0].copy_(last)
         with torch.cuda.device(dev):
             status = library.peco_kmeans_iterate(
                 _native.ptr(p.x), p.x.stride(0), _native.ptr(p.init), _native.ptr(centers[0]), _native.ptr(centers[1]),
                 _native.ptr(labels), _native.ptr(counts), _native.ptr(indices), _native.ptr(offsets), p.batch, p.tokens,
-                p.clusters, dims, _DTYPES[p.x.dtype], done, step, _float32_floor(tol), _native.ptr(flags), _native.ptr(ws),
-                ws_bytes, _retain_on_current_stream(dev, p.x, p.init))
+                p.clusters, dims, _DTYPES[p.x.dtype], done, step, tol, _native.ptr(flags[at]), _native.ptr(ws), ws_bytes,
+                _retain_on_current_stream(dev, p.x, p.init))
         _raise_cluster_error(status)
-        last = flags[step]
-        moved = flags[1:, 0].tolist()  # waits for these iterations
+        moved = [row[0] for row in flags[at + 1:at + 1 + step].tolist()]  # waits for these iterations
+        at += step
         done += moved.index(0) + 1 if 0 in moved else step
         if 0 in moved:
             break

@@ -112,9 +112,10 @@ struct KmIter {
     int32_t* hist[kMaxKm];     // nullable: tile histograms the assign adds its labels to
     float* screen;             // kDump assignments only: screened distances [batch, tokens, K]
     // Fits that stop at convergence only (else null): row [1 + batch] of the iteration before
-    // (prev) and of this one (cur), {some centre moved past tol, entry b changed at all}. An
-    // iteration after one that moved nothing past tol does nothing; an entry whose centres came out
-    // bit for bit as they went in is at its fixed point and is skipped (skip_fixed) from then on.
+    // (prev, null for the first one) and of this one (cur), {some centre moved past tol, entry b
+    // changed at all}. An iteration after one that moved nothing past tol does nothing; an entry whose
+    // centres came out bit for bit as they went in is at its fixed point and is skipped (skip_fixed)
+    // from then on.
     const int32_t* prev;
     int32_t* cur;
     float tol;
@@ -1037,12 +1038,12 @@ __global__ __launch_bounds__(kUpdateWaves * kWave) void km_update_kernel(KmArgs 
     }
     const int count = end - begin;
     const int64_t cbase = static_cast<int64_t>(cl) * D + lane * PER;
-    float moved = 0.0f;     // squared displacement of this lane's channels (with it.prev)
+    float moved = 0.0f;     // squared displacement of this lane's channels (with it.cur)
     bool changed = false;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
         const float mean = count > 0 ? s[i] / static_cast<float>(count) : it.src[p][cbase + i];
-        if (it.prev) {
+        if (it.cur) {
             const float before = it.src[p][cbase + i];
             const float step = mean - before;
             moved = fmaf(step, step, moved);
@@ -1057,7 +1058,7 @@ __global__ __launch_bounds__(kUpdateWaves * kWave) void km_update_kernel(KmArgs 
         P.prep_hi[cbase + i] = hi;
         P.prep_lo[cbase + i] = lo;
     }
-    if (it.prev) {
+    if (it.cur) {
 #pragma unroll
         for (int m = 1; m < kWave; m <<= 1) moved += __shfl_xor(moved, m, kWave);
         const bool any_changed = __any(changed);
@@ -1440,7 +1441,7 @@ KmFitDesc slice_desc(const KmFitDesc& d, int b0, int nb, int dims, int dtype) {
 
 // Iterations [first, first + iterations) of a fit that stops at convergence (one problem): means of
 // iteration i go to centers[i % 2], flags [iterations + 1, 1 + batch] as KmIter::prev (row 0: the
-// iteration before the first one).
+// iteration before the first one of the call, unused for the first of the fit).
 struct KmTolRun {
     int first;
     float tol;
@@ -1655,7 +1656,7 @@ hipError_t km_fit_launches(const KmFitDesc* descs, int num, int dims, int dtype,
         iters[i].sq_mode = n == 0 ? 1 : 2;
         if (run) {
             const int64_t row = 1 + a.p[0].batch;
-            iters[i].prev = run->flags + i * row;
+            iters[i].prev = n == 0 ? nullptr : run->flags + i * row;
             iters[i].cur = run->flags + (i + 1) * row;
             iters[i].tol = run->tol;
             // An unchanged entry's centres are in both buffers only from the second iteration on.

@@ -63,3 +63,37 @@ def test_tolerance_is_rounded_down_to_float32():
     for value in (0.1, 1e-4, 1.0, 1e300, 5e-46, math.pi):
         f = clustering_cuda._float32_floor(value)
         assert f <= value and torch.nextafter(torch.tensor(f), torch.tensor(float("inf"))).double().item() > value
+
+
+@pytest.mark.parametrize("max_iters", [1, 2, 3, 6, 7, 14, 15, 63, 64, 65, 150])
+def test_fit_that_never_settles_runs_every_iteration(max_iters):
+    """Every length of the last stretch between looks, and more iterations than one block of flags."""
+    g = torch.Generator().manual_seed(5)
+    x = torch.randn(2, 300, 64, generator=g).to(DEV)
+    init = x[:, :4].contiguous()
+    init[1, 2, 0] = float("nan")
+    got, ref = (f(x, *a) for f, a in ((clustering.fit_token_clusters, (4, max_iters, 1e-4, init)),
+                                      (_stepwise, (init, max_iters, 1e-4))))
+    assert got[3] == ref[3] == max_iters
+    assert torch.equal(got[0], ref[0]) and torch.equal(got[2], ref[2])
+    assert torch.equal(got[1].nan_to_num(7.0), ref[1].nan_to_num(7.0))
+
+
+def test_fit_from_its_fixed_point_launches_little(monkeypatch):
+    """A fit that stops at once does not first launch the iterations of a long one."""
+    g = torch.Generator().manual_seed(3)
+    x = torch.randn(2, 500, 64, generator=g).to(DEV)
+    settled = clustering.fit_token_clusters(x, 6, 200, 1e-4, x[:, :6].contiguous())[1]
+    library, launched = clustering_cuda._library(), []
+
+    class Counting:
+        def __getattr__(self, name):
+            return getattr(library, name)
+
+        def peco_kmeans_iterate(self, *args):
+            launched.append(args[15])
+            return library.peco_kmeans_iterate(*args)
+
+    monkeypatch.setattr(clustering_cuda, "_library", Counting)
+    assert clustering.fit_token_clusters(x, 6, 50, 1e-4, settled)[3] == 1
+    assert sum(launched) <= 2
