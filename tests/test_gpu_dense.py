@@ -1,7 +1,8 @@
 """Dense attention of the warm-up branch (processor.dense_attention) on the sparse kernel: lengths at
 the edges of its key tiles, row blocks and items, both item sizes, the persistent grid, layouts,
 and the calls that stay with SDPA. The reference is float32 softmax attention per segment; bounds
-are those of the attention tests (P and the output are rounded to 16 bits)."""
+are those of the attention tests (P and the output are rounded to 16 bits) and, per segment, one on the
+error relative to the result, which a single key too many or too few would pass (``_check``)."""
 import pytest
 import torch
 
@@ -19,6 +20,20 @@ def _reference(q, k, v, valid):
                 s = q[:, h, a:b].float() @ k[:, h, a:b].float().transpose(1, 2).contiguous() * q.shape[3] ** -0.5
                 out[:, h, a:b] = torch.softmax(s, -1) @ v[:, h, a:b].float()
     return out
+
+
+def _check(out, ref, valid, dtype):
+    """Per segment of n keys the 2-norm of the error is at most 2^-7.5 (bf16) or 2^-10.5 (fp16) of the
+    result's: rounding the weights and the output to u = 2^-9 or 2^-12 of themselves costs each element
+    an independent error of about u / sqrt(3) of the row's size each, 0.8 u together; the bound is 2.8 u =
+    5.5e-3 or 6.9e-4. One key more or less moves a row of normal values by 1 / sqrt(n) of its size: 1.1e-2 at
+    the longest 8192 keys here. The smallest fp16 subnormal is allowed for beside it."""
+    err = (out.float() - ref)
+    assert err.abs().max().item() <= 2e-2 and err.abs().mean().item() <= 2e-3
+    bound = 2.0 ** -7.5 if dtype == torch.bfloat16 else 2.0 ** -10.5
+    for part in (slice(0, valid), slice(valid, ref.shape[2])):
+        n = ref[:, :, part].numel()
+        assert err[:, :, part].norm().item() <= bound * ref[:, :, part].norm().item() + 2.0 ** -25 * n ** 0.5, part
 
 
 def _inputs(batch, heads, length, dim, dtype):
@@ -43,8 +58,15 @@ def test_dense_attention_matches_reference(dtype, batch, heads, length, dim, val
     assert attention_cuda.dense_supported(q, k, v, valid)
     ref = _reference(q, k, v, valid)
     for _ in range(2):  # the second call finds the workspace as the first left it
-        err = (processor.dense_attention(q, k, v, valid).float() - ref).abs()
-        assert err.max().item() <= 2e-2 and err.mean().item() <= 2e-3
+        _check(processor.dense_attention(q, k, v, valid), ref, valid, dtype)
+    # The bound sees one key of the longer segment moved to the other side of the boundary.
+    if length > 64 and 0 < valid < length:
+        moved = valid - 1 if valid > length - valid else valid + 1
+        wrong = _reference(q[:, :2], k[:, :2], v[:, :2], moved)
+        edge = min(valid, moved)
+        for part in (slice(0, edge), slice(max(valid, moved), length)):
+            if part.stop - part.start > 1:
+                assert (wrong[:, :, part] - ref[:, :2, part]).norm() > 2.0 ** -7.5 * ref[:, :2, part].norm()
 
 
 @pytest.mark.parametrize("heads,length,dim,valid", [
@@ -52,8 +74,7 @@ def test_dense_attention_matches_reference(dtype, batch, heads, length, dim, val
 def test_dense_attention_short_items(heads, length, dim, valid):
     """Items of 64 rows, of one row and past a whole tile, few and many per head."""
     q, k, v = _inputs(1, heads, length, dim, torch.bfloat16)
-    err = (processor.dense_attention(q, k, v, valid).float() - _reference(q, k, v, valid)).abs()
-    assert err.max().item() <= 2e-2 and err.mean().item() <= 2e-3
+    _check(processor.dense_attention(q, k, v, valid), _reference(q, k, v, valid), valid, torch.bfloat16)
 
 
 def test_dense_attention_keeps_layout_and_sdpa_calls():
