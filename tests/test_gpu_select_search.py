@@ -55,16 +55,21 @@ def test_select_ties_across_blocks_match_oracle(ck, m):
 
 @pytest.mark.parametrize("poison", [float("nan"), float("inf")])
 def test_select_non_finite_row_leaves_the_others(poison):
-    """A query centroid that is not finite: its own row still keeps at least the minimum, every other
-    row and the padding columns are the oracle's."""
+    """A query centroid that is not finite: every other row is the oracle's. Its own row, which takes the
+    sequential walk, keeps exactly the minimum when no probability is a number (by index); with an
+    infinite centroid the keys of infinite mass have the probability inf / inf, ordered last, and all
+    keys of zero mass come before them and are kept."""
     qc, kc, qs, ks = _case(5, 2, 12, 300, 128)
     qs.clamp_(min=1)
-    ref = reference_path.select_connections(qc, kc, qs, ks, 0.8, 0.0)
+    ref = reference_path.select_connections(qc, kc, qs, ks, 0.8, 5 / 300)
     qc[0, 1, 7, 3] = poison
     got, _, _ = clustering_cuda.select_connections(qc.to(DEV), kc.to(DEV), qs.to(DEV), ks.to(DEV), 0.8, 5)
-    ref5 = reference_path.select_connections(qc[:, :1], kc[:, :1], qs[:, :1], ks[:, :1], 0.8, 5 / 300)
     got = got.cpu()
-    assert torch.equal(got[:, :1], ref5)
     rows = [r for r in range(12) if r != 7]
-    assert (got[0, 1, rows].int() >= ref[0, 1, rows].int()).all()
-    assert got[0, 1, 7].sum() <= (ks[0, 1] > 0).sum()
+    assert torch.equal(got[:, :1], ref[:, :1]) and torch.equal(got[0, 1, rows], ref[0, 1, rows])
+    want = (ks[0, 1] > 0) & (kc[0, 1, :, 3] < 0)
+    if poison != poison:
+        want = torch.zeros(300, dtype=torch.bool)
+        want[(ks[0, 1] > 0).nonzero()[:5, 0]] = True
+        assert torch.equal(want, reference_path.select_connections(qc, kc, qs, ks, 0.8, 5 / 300)[0, 1, 7])
+    assert want.sum() >= 5 and torch.equal(got[0, 1, 7], want)
