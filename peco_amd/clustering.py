@@ -62,6 +62,13 @@ def fit_token_clusters(x, n_clusters, max_iters=100, tol=1e-4, init_centroids=No
     return clustering_cuda.kmeans_fit_until(clustering_cuda.KMeansProblem(x, centers), max_iters, tol)
 
 
+# Longest entry whose labels are sorted by label_argsort. Its time depends on the range of the labels, which
+# only the device knows: up to 4M different values it wins at every length (us, 300 clusters, against
+# torch.argsort: 24 x 118800 55 and 250, 1 x 1000000 128 and 189), but labels that span more are
+# sorted by one workgroup per entry, whose time grows with the length (1 x 1000000 10.6 ms).
+_ARGSORT_TOKENS = 131072
+
+
 def _prepare_sequence_indices(tensor, labels, dim, sorted_indices):
     """Validate token reordering and return contiguous int32 indices [BH,N] (peco/clustering.py:92-108)."""
     if tensor.ndim != 4 or dim not in (2, -2):
@@ -76,7 +83,8 @@ def _prepare_sequence_indices(tensor, labels, dim, sorted_indices):
             raise ValueError("labels must contain one cluster ID per token on the same device")
         # Stable sort keeps the original order inside each cluster.
         rows = labels.reshape(batch * heads, tokens)
-        if rows.is_cuda and rows.dtype in (torch.int32, torch.int64) and _native.plain_tensors(rows):
+        if rows.is_cuda and rows.dtype in (torch.int32, torch.int64) and tokens <= _ARGSORT_TOKENS and \
+                _native.plain_tensors(rows):
             return clustering_cuda.label_argsort(rows)
         sorted_indices = torch.argsort(rows, dim=-1, stable=True)
     if sorted_indices.numel() != batch * heads * tokens or sorted_indices.device != tensor.device:

@@ -35,3 +35,17 @@ def test_gather_by_labels_takes_any_label_tensor():
         assert indices.dtype == torch.int32 and torch.equal(indices.cpu().long(), want)
         assert torch.equal(packed.cpu(), x.cpu().gather(2, want[None, ..., None].expand(-1, -1, -1, 64)))
         assert torch.equal(clustering.restore_sequence_order(packed, indices), x)
+
+
+def test_gather_by_labels_of_very_long_entries_stays_with_torch(monkeypatch):
+    """The argsort's time on labels of any value grows with the length of an entry."""
+    calls = []
+    monkeypatch.setattr(clustering_cuda, "label_argsort", lambda rows: calls.append(rows.shape))
+    for tokens, taken in ((131072, True), (131073, False), (1000000, False)):
+        x = torch.zeros(1, 1, tokens, 8, dtype=torch.bfloat16, device=DEV)
+        labels = torch.arange(tokens, device=DEV).flip(0) * (2**20 + 1)
+        calls.clear()
+        indices = clustering._prepare_sequence_indices(x, labels, 2, None)
+        assert bool(calls) == taken
+        if not taken:
+            assert indices.dtype == torch.int32 and torch.equal(indices[0], torch.arange(tokens, device=DEV).flip(0).int())
