@@ -960,8 +960,11 @@ __device__ __forceinline__ void pack_text_rows(const KmArgs& a, int block) {
 }
 
 // kPack: 0 plain update; 1 the last update of a fit that packs some problem in cluster order
-// (those problems' members are packed by the update itself).
-template <int DT, int D, int kPack = 0>
+// (those problems' members are packed by the update itself). kConverge: an iteration of a fit that
+// stops at convergence, which skips settled entries and flags what moved (KmIter::prev, cur). As a
+// runtime branch that cost every other fit's launch 0.4-0.7 us of 6-16 (256 centres of 2000 to 40000
+// tokens).
+template <int DT, int D, int kPack = 0, bool kConverge = false>
 __global__ __launch_bounds__(kUpdateWaves * kWave) void km_update_kernel(KmArgs a, KmIter it) {
     constexpr int PER = D / kWave;  // channels per lane (1 or 2)
     __shared__ float row[kUpdateWaves][D];
@@ -983,7 +986,9 @@ __global__ __launch_bounds__(kUpdateWaves * kWave) void km_update_kernel(KmArgs 
     if (cl >= P.batch * K) return;  // wave mode only: the last workgroup may be partial
     const int b = cl / K;
     const int j = cl % K;
-    if (km_settled(it.prev, it.skip_fixed, b)) return;
+    if constexpr (kConverge) {
+        if (km_settled(it.prev, it.skip_fixed, b)) return;
+    }
     const int32_t* off = P.offsets + static_cast<int64_t>(b) * (K + 1);
     const int begin = off[j], end = off[j + 1];
     const int32_t* idx = P.indices + static_cast<int64_t>(b) * P.tokens;
@@ -1038,12 +1043,12 @@ __global__ __launch_bounds__(kUpdateWaves * kWave) void km_update_kernel(KmArgs 
     }
     const int count = end - begin;
     const int64_t cbase = static_cast<int64_t>(cl) * D + lane * PER;
-    float moved = 0.0f;     // squared displacement of this lane's channels (with it.cur)
+    float moved = 0.0f;     // kConverge: squared displacement of this lane's channels
     bool changed = false;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
         const float mean = count > 0 ? s[i] / static_cast<float>(count) : it.src[p][cbase + i];
-        if (it.cur) {
+        if constexpr (kConverge) {
             const float before = it.src[p][cbase + i];
             const float step = mean - before;
             moved = fmaf(step, step, moved);
@@ -1058,7 +1063,7 @@ __global__ __launch_bounds__(kUpdateWaves * kWave) void km_update_kernel(KmArgs 
         P.prep_hi[cbase + i] = hi;
         P.prep_lo[cbase + i] = lo;
     }
-    if (it.cur) {
+    if constexpr (kConverge) {
 #pragma unroll
         for (int m = 1; m < kWave; m <<= 1) moved += __shfl_xor(moved, m, kWave);
         const bool any_changed = __any(changed);
@@ -1288,6 +1293,9 @@ hipError_t run_fit(KmArgs& a, const KmIter* iters, int first, int iterations, So
         }
         if (i + 1 == iterations && cluster_order)
             hipLaunchKernelGGL((km_update_kernel<DT, D, 1>), dim3(a.total_upd_blocks + a.text_blocks),
+                               dim3(kUpdateWaves * kWave), 0, s, a, iters[i]);
+        else if (iters[i].cur)
+            hipLaunchKernelGGL((km_update_kernel<DT, D, 0, true>), dim3(a.total_upd_blocks),
                                dim3(kUpdateWaves * kWave), 0, s, a, iters[i]);
         else
             hipLaunchKernelGGL((km_update_kernel<DT, D>), dim3(a.total_upd_blocks), dim3(kUpdateWaves * kWave), 0, s,
