@@ -199,10 +199,11 @@ def plain_tensors(*tensors) -> bool:
 
     if torch.compiler.is_compiling():
         return False
+    dual = torch.autograd.forward_ad._current_level >= 0  # (no tensor has a tangent outside a level)
     for t in tensors:
         if type(t) not in (torch.Tensor, torch.nn.Parameter) or torch._C._functorch.is_functorch_wrapped_tensor(t):
             return False
-        if torch.autograd.forward_ad.unpack_dual(t).tangent is not None:
+        if dual and torch.autograd.forward_ad.unpack_dual(t).tangent is not None:
             return False
     return True
 

@@ -166,11 +166,24 @@ def _rotary_tables(fn, freqs, rows, dim, device):
     return tuple(freqs)
 
 
+# Elements up to which a projection without rotation is left to torch: the placing launch costs the host
+# about 10 us more with its checks, and a call of that size waits for the host. A copy of 8M elements takes the device
+# 15 us, the launch 6.5; a norm and copy of 1M 11 and 3 (bf16). Prologue of a call without rotation, the
+# host's time, 24 heads x 1024 + 32 rows: 250 us, 335 with the launch.
+_COPY_ELEMENTS = 1 << 23
+_NORM_ELEMENTS = 1 << 20
+
+
+def _fits(part, buffer):
+    """Whether shapes and dtype of ``part`` [B, H, rows, D] agree with ``buffer`` [3, B, H, S, D]'s."""
+    return part.shape[:2] == buffer.shape[1:3] and part.shape[3] == buffer.shape[4] and \
+        part.dtype == buffer.dtype and _native.plain_tensors(buffer)
+
+
 def _placeable(part, buffer):
     """Whether place_heads takes ``part`` [B, H, rows, D] into ``buffer`` [3, B, H, S, D] (None: any that
     fits): the shapes and dtype agree and its rows start on 16 bytes with adjacent channels."""
-    if buffer is not None and (part.shape[:2] != buffer.shape[1:3] or part.shape[3] != buffer.shape[4] or
-                               part.dtype != buffer.dtype or not _native.plain_tensors(buffer)):
+    if buffer is not None and not _fits(part, buffer):
         return False
     return part.shape[3] in (64, 128) and part.shape[2] > 0 and part.dtype in (torch.bfloat16, torch.float16) and \
         part.is_cuda and part.stride(3) == 1 and all(s % 8 == 0 for s in part.stride()[:3]) and \
@@ -386,9 +399,14 @@ class PecoAttention:
                 part = proj(source).unflatten(2, (attn.heads, -1)).transpose(1, 2)  # [B, H, rows, D] view
                 norm = norms[slot] if slot < 2 else None
                 turn = slot < 2 and freqs is not None
-                tables = _rotary_tables(rotary, freqs, rows, part.shape[3], part.device) if turn else None
-                turn = turn and tables is None  # by torch
-                rms = None if norm is None or turn or not _placeable(part, None) else _rms_norm(norm, part)
+                large = part.numel() > (_COPY_ELEMENTS if norm is None else _NORM_ELEMENTS)
+                place = (turn or large) and _placeable(part, None)
+                projected, tables, rms = part, None, None
+                if place and turn:
+                    tables = _rotary_tables(rotary, freqs, rows, part.shape[3], part.device)
+                    turn = tables is None  # by torch
+                if place and norm is not None and not turn:
+                    rms = _rms_norm(norm, part)
                 if norm is not None and rms is None:
                     # The rows as projected, where the norm cannot tell: no copy into head order first.
                     swap = part.is_cuda and _per_channel_norm(norm)
@@ -398,7 +416,8 @@ class PecoAttention:
                 if qkv is None:
                     batch, heads, _, dim = part.shape
                     qkv = torch.empty((3, batch, heads, length, dim), dtype=part.dtype, device=part.device)
-                if _placeable(part, qkv):
+                place = place and (tables is not None or rms is not None or part.numel() > _COPY_ELEMENTS)
+                if place and (part is projected or _placeable(part, None)) and _fits(part, qkv):
                     clustering_cuda.place_heads(part, qkv[slot], first, tables, rms)
                 else:
                     part = part if rms is None else norm(part)

@@ -103,8 +103,9 @@ def test_call_matches_the_torch_prologue(double, text, monkeypatch):
 
 
 @pytest.mark.parametrize("eps,size", [(0.0, 1e-20), (0.0, 3e-19), (1e-40, 1e-20), (2.0 ** -126, 1e-20), (1e-6, 1.0)])
-def test_call_with_a_norm_of_tiny_rows(eps, size):
+def test_call_with_a_norm_of_tiny_rows(eps, size, monkeypatch):
     """Rows whose mean square is subnormal come out as the block's norm gives them, whatever its eps."""
+    monkeypatch.setattr(processor, "_NORM_ELEMENTS", 0)  # the placing launch for any size
     heads, dim, video = 3, 64, 40
     torch.manual_seed(6)
     block = _Block(heads, dim, False).to(DEV, torch.bfloat16)
@@ -121,3 +122,28 @@ def test_call_with_a_norm_of_tiny_rows(eps, size):
         rows = getattr(block, "to_" + name)(hidden).unflatten(2, (heads, -1))
         want = getattr(block, "norm_" + name)(rows)
         assert torch.isfinite(want).all() and torch.equal(got[..., at:at + dim], want)
+
+
+@pytest.mark.parametrize("rotate", [False, True])
+@pytest.mark.parametrize("norm", [None, torch.nn.RMSNorm, torch.nn.LayerNorm])
+def test_call_is_the_same_on_both_sides_of_the_size_rules(norm, rotate, monkeypatch):
+    """A projection placed by torch operations and by the placing launch: the same bits."""
+    heads, dim, video, text = 5, 128, 67, 9
+    torch.manual_seed(8)
+    block = _Block(heads, dim, False).to(DEV, torch.bfloat16)
+    block.norm_q, block.norm_k = (norm(dim, eps=1e-6).to(DEV, torch.bfloat16) if norm else None for _ in range(2))
+    g = torch.Generator().manual_seed(3)
+    hidden, enc = (torch.randn(2, rows, heads * dim, generator=g).to(DEV, torch.bfloat16) for rows in (video, text))
+    freqs = _tables(video, dim, g) if rotate else None
+    layer = processor.PecoAttention(0, processor.PecoConfig(), processor.InferenceContext(5, text, text))
+    layer.attention = lambda q, k, v: torch.cat((q, k, v), -1)
+    placed, outs = [], []
+    launch = clustering_cuda.place_heads
+    monkeypatch.setattr(clustering_cuda, "place_heads", lambda *a: (placed.append(a), launch(*a)))
+    for limit in (0, 1 << 40):
+        monkeypatch.setattr(processor, "_COPY_ELEMENTS", limit)
+        monkeypatch.setattr(processor, "_NORM_ELEMENTS", limit)
+        placed.clear()
+        outs.append(layer(block, hidden, enc, image_rotary_emb=freqs))
+        assert len(placed) == (6 if limit == 0 else 2 * rotate)
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
