@@ -166,10 +166,11 @@ def _rotary_tables(fn, freqs, rows, dim, device):
     return tuple(freqs)
 
 
-# Elements up to which a projection without rotation is left to torch: the placing launch costs the host
-# about 10 us more with its checks, and a call of that size waits for the host. A copy of 8M elements takes the device
-# 15 us, the launch 6.5; a norm and copy of 1M 11 and 3 (bf16). Prologue of a call without rotation, the
-# host's time, 24 heads x 1024 + 32 rows: 250 us, 335 with the launch.
+# Elements of a projection over the whole sequence up to which its rows are left to torch where no rotation
+# is applied: the placing launch costs the host about 10 us more with its checks, and a call of that size
+# waits for the host (prologue without rotation, 24 heads x 1024 + 32 rows of 128 channels: 250 us, 335 with
+# the launch), while a longer one waits for the device (a copy of 8M 16-bit elements 15 us against 6.5, a
+# norm and a copy of 1M 11 against 3: the text rows of 24 heads x 6750 + 256 by torch, 1.5% of the call).
 _COPY_ELEMENTS = 1 << 23
 _NORM_ELEMENTS = 1 << 20
 
@@ -399,8 +400,8 @@ class PecoAttention:
                 part = proj(source).unflatten(2, (attn.heads, -1)).transpose(1, 2)  # [B, H, rows, D] view
                 norm = norms[slot] if slot < 2 else None
                 turn = slot < 2 and freqs is not None
-                large = part.numel() > (_COPY_ELEMENTS if norm is None else _NORM_ELEMENTS)
-                place = (turn or large) and _placeable(part, None)
+                size = part.numel() // max(rows, 1) * length
+                place = (turn or size > (_COPY_ELEMENTS if norm is None else _NORM_ELEMENTS)) and _placeable(part, None)
                 projected, tables, rms = part, None, None
                 if place and turn:
                     tables = _rotary_tables(rotary, freqs, rows, part.shape[3], part.device)
@@ -416,7 +417,7 @@ class PecoAttention:
                 if qkv is None:
                     batch, heads, _, dim = part.shape
                     qkv = torch.empty((3, batch, heads, length, dim), dtype=part.dtype, device=part.device)
-                place = place and (tables is not None or rms is not None or part.numel() > _COPY_ELEMENTS)
+                place = place and (tables is not None or rms is not None or size > _COPY_ELEMENTS)
                 if place and (part is projected or _placeable(part, None)) and _fits(part, qkv):
                     clustering_cuda.place_heads(part, qkv[slot], first, tables, rms)
                 else:
