@@ -1702,8 +1702,8 @@ PECO_API size_t peco_kmeans_workspace_size(int batch, int tokens, int clusters, 
 }
 
 // Fused fit of one or two independent problems (e.g. Q with KQ centres and K with KK
-// centres), the second on a library stream forked from and joined to `stream`. Problem i is
-// described by the i-th element of each array.
+// centres), a large one as four chains of launches forked from and joined to `stream`
+// (km_fit_chains). Problem i is described by the i-th element of each array.
 PECO_API int peco_kmeans_fit(int num_problems, const void* const* x, const int64_t* x_batch_stride,
                              const float* const* centers_in,
                              float* const* centers_out, int32_t* const* labels, int32_t* const* counts,
@@ -1729,7 +1729,7 @@ PECO_API int peco_kmeans_fit(int num_problems, const void* const* x, const int64
 // Iterations of a fit that stops at convergence (peco/clustering.py:61-86 with tol > 0), without a
 // host round trip per iteration: the update flags whether a centre moved past tol, later launches
 // return at once when none did, and entries at their fixed point are skipped. 24 x 6750 x 128 fp32
-// rows, 100 centres, about 45 iterations: 1.7 ms; one fit call, a norm, a maximum and a copy to the
+// rows, 100 centres, 24 iterations: 1.7 ms; one fit call, a norm, a maximum and a copy to the
 // host per iteration took 3.8 ms.
 PECO_API int peco_kmeans_iterate(const void* x, int64_t x_batch_stride, const float* centers_in, float* centers_a,
                                  float* centers_b, int32_t* labels, int32_t* counts, int32_t* sorted_indices,
